@@ -22,8 +22,11 @@
 //                  LDS ring, a running argmax per column stream (gemm_lmhead: A resident in LDS)
 //   gemm_large_m   4 waves x 16 columns, 64 rows per block; the A tile of each k-block is
 //                  staged once in LDS in MFMA fragment order, the next k-block's loads in
-//                  flight meanwhile (batched lanes);
+//                  flight meanwhile (batched lanes: k-block chains, and operands the others
+//                  cannot take);
 //                  a non-plain producer runs first as its own elementwise kernel
+//   gemm_ksplit    stored outputs, K != 1024, few tiles: 32-row blocks whose waves split K
+//   gemm_rows64    stored outputs from row-major A, more tiles: 64 x 128 blocks, an LDS ring
 // kEPartial (N = 1024 outputs feeding the residual add): each block computes ONE k-block
 // chain and stores it to kpart[kb][M][N]; the following add+norm kernel sums the chains in
 // k-block order. That keeps ~KB x more blocks in flight without cross-block atomics.
@@ -913,6 +916,43 @@ __global__ void __launch_bounds__(512) gemm_wide(GemmArgs a) {
     }
 }
 
+// Epilogue of a 64 x 128 block whose 8 waves hold 32 x 32 outputs each (gemm_wide64,
+// gemm_rows64): the wave's two row tiles start at row0; the block's ring is drained.
+template <int EM>
+__device__ __forceinline__ void store_wide64(const GemmArgs& a, const q35_f32x4 (&sum)[2][2], int row0, int nblk,
+                                             uint16_t* wl, int wv, int lane) {
+    const int wn = wv & 3, ntiles = a.N / 16, half = a.N / 32;
+    if (EM == kESiluMul) {
+        uint16_t* ob = wl + (size_t)wv * 512;                        // [32 rows][16 cols]
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                ob[(i * 16 + 4 * (lane >> 4) + r) * 16 + (lane & 15)] =
+                    f2bf(__fmul_rn(rbf(silu_f(rbf(sum[i][0][r]))), rbf(sum[i][1][r])));
+        wave_sync();
+        const int row = lane >> 1, piece = lane & 1, jt = nblk * 4 + wn, grow = row0 + row;
+        if (grow < a.M && jt < half)
+            *(q35_u32x4*)(a.Y + (size_t)grow * a.ldy + jt * 16 + piece * 8) = *(const q35_u32x4*)(ob + row * 16 + piece * 8);
+        return;
+    }
+    uint16_t* ob = wl + (size_t)wv * 1024;                           // [32 rows][32 cols]
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int jn = 0; jn < 2; ++jn)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ob[(i * 16 + 4 * (lane >> 4) + r) * 32 + jn * 16 + (lane & 15)] = f2bf(sum[i][jn][r]);
+    wave_sync();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int ch = lane + 64 * q, row = ch >> 2, piece = ch & 3;
+        const int nt = nblk * 8 + wn * 2 + (piece >> 1), grow = row0 + row;
+        if (grow < a.M && nt < ntiles)
+            *(q35_u32x4*)(a.Y + (size_t)grow * a.ldy + nt * 16 + (piece & 1) * 8) = *(const q35_u32x4*)(ob + row * 32 + piece * 8);
+    }
+}
+
 // K = 1024 at batched lanes (M <= 511 rows, decode): gemm_wide's ring and pipeline with 64-row x
 // 128-column block tiles (224 blocks for gate|up at 256 rows). kEPartial: any K (a multiple of
 // 512), all of K in the block and the k-block chains summed in order into chain 0 -- the
@@ -1035,35 +1075,238 @@ __global__ void __launch_bounds__(512) gemm_wide64(GemmArgs a) {
         return;
     }
     __syncthreads();                   // the ring is drained by every wave: wave-private staging
-    uint16_t* wl = (uint16_t*)dyn_lds;
-    if (EM == kESiluMul) {
-        uint16_t* ob = wl + (size_t)wv * 512;                        // [32 rows][16 cols]
+    store_wide64<EM>(a, sum, row0, nblk, (uint16_t*)dyn_lds, wv, lane);
+}
+
+// ---------------------------------------------------------------- row-major A, any K
+// gemm_wide64 for callers whose A is plain rows: 64 x 128 blocks of 8 waves (32 x 32 each), the
+// K stream through a ring of three 48 KiB stages of four MFMA steps (half a k-block) instead of
+// six of two: a stage then holds 64 contiguous bytes of each (row, 64-wide k-group), so the DMA
+// reads A straight from its rows in 64-byte pieces and no pass re-tiles it first. One DMA
+// instruction fills the KiB of (row tile, k-group g): lane j reads chunk (j & 3) ^ ((j >> 3) & 3)
+// of row j >> 2, and the fragment of (row r, step s) is at r * 64 + ((s ^ ((r >> 1) & 3)) * 16):
+// 8 consecutive rows then cover all banks. Two stages (96 KiB) in flight while one is computed,
+// its fragments in registers a stage ahead. Bound by the CU's LDS (a stage is 128 KiB of fragment
+// reads and 48 KiB of DMA writes against 512 cycles of MFMA): down_proj (K = 3584, N = 1024) at
+// 1,999 rows 24.8 us = 591 TFLOP/s, 35.1 in gemm_large_m's 64 x 64 blocks. Canonical reduction.
+constexpr int kRowsRing = 3;
+constexpr int kRowsStage = 48 * 1024;
+constexpr int kRowsLds = kRowsRing * kRowsStage;    // 144 KiB
+
+template <int EM>
+__global__ void __launch_bounds__(512) gemm_rows64(GemmArgs a) {
+    extern __shared__ q35_u32x4 dyn_lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wv >> 2, wn = wv & 3;
+    const int mb = (a.M + 63) / 64;
+    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+    const int ntiles = a.N / 16, half = a.N / 32;
+    const int ncb = EM == kESiluMul ? (half + 3) / 4 : (ntiles + 7) / 8;
+    // at most 8 column blocks: row blocks by XCD (each XCD fetches its rows of A and all of W),
+    // else column blocks by XCD (its slab of W and all of A)
+    const bool byrow = ncb <= 8;
+    const int nblk = byrow ? idx % ncb : (idx / mb) * 8 + xcd;
+    const int rb = byrow ? (idx / ncb) * 8 + xcd : idx % mb;
+    if (rb >= mb || nblk >= ncb) return;
+    const int KB = a.K >> 8, NS = 2 * KB;
+    // DMA pieces of a stage: wave wv fills A pieces 2 wv, 2 wv + 1 (row tile wv / 2, k-groups
+    // 2 (wv % 2), + 1) and the four steps of column tile wv; rows and tiles past the end re-read
+    // the last valid one (they feed outputs that are not stored)
+    const char* abase = (const char*)((const uint16_t*)a.X + (size_t)rb * 64 * a.ldx);
+    const int jr = lane >> 2;
+    const int arow = min(rb * 64 + (wv >> 1) * 16 + jr, a.M - 1) - rb * 64;
+    const unsigned aoff = (unsigned)arow * (unsigned)a.ldx * 2u + (unsigned)(((lane & 3) ^ ((jr >> 1) & 3)) * 16 + (wv & 1) * 256);
+    const int ct = EM == kESiluMul ? (wv < 4 ? min(nblk * 4 + wv, half - 1) : half + min(nblk * 4 + wv - 4, half - 1))
+                                   : min(nblk * 8 + wv, ntiles - 1);
+    const char* wbase = (const char*)(a.W + (size_t)ct * KB * 4096);
+    auto issue = [&](int j) {          // stage j: k-block j / 2, steps 4 (j % 2) .. + 3
+        char* lds = (char*)dyn_lds + (j % kRowsRing) * kRowsStage;
+        const char* ap = uniform_ptr(abase + (size_t)j / 2 * 512 + (j & 1) * 64);
 #pragma unroll
         for (int i = 0; i < 2; ++i)
+            __builtin_amdgcn_global_load_lds((const void*)(ap + i * 128 + aoff),
+                                             (__attribute__((address_space(3))) void*)(lds + (2 * wv + i) * 1024), 16, 0, 0);
+        const char* wp = uniform_ptr(wbase + (size_t)j * 4096);
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                ob[(i * 16 + 4 * (lane >> 4) + r) * 16 + (lane & 15)] =
-                    f2bf(__fmul_rn(rbf(silu_f(rbf(sum[i][0][r]))), rbf(sum[i][1][r])));
-        wave_sync();
-        const int row = lane >> 1, piece = lane & 1, jt = nblk * 4 + wn, grow = row0 + row;
-        if (grow < a.M && jt < half)
-            *(q35_u32x4*)(a.Y + (size_t)grow * a.ldy + jt * 16 + piece * 8) = *(const q35_u32x4*)(ob + row * 16 + piece * 8);
-        return;
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_global_load_lds((const void*)(wp + i * 1024 + lane * 16),
+                                             (__attribute__((address_space(3))) void*)(lds + 16384 + (4 * wv + i) * 1024), 16, 0, 0);
+    };
+    const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) const void*)dyn_lds;
+    const int r16 = lane & 15;
+    unsigned aaddr[4];                 // this lane's fragment of row tile 2 wm at step s
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+        aaddr[s] = lds0 + (unsigned)(wm * 8192 + (lane >> 4) * 1024 + r16 * 64 + ((s ^ ((r16 >> 1) & 3)) * 16));
+    const unsigned baddr = lds0 + 16384u + (unsigned)((EM == kESiluMul ? 1 : 2) * wn * 4096) + lane * 16;
+    constexpr int B1 = EM == kESiluMul ? 16384 : 4096;                // offset of the second B tile
+    q35_u32x4 fa[2][4][2], fb[2][4][2];                               // [set][step][tile]
+#define Q35_WRD(dst, base, off) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(base), "n"(off) : "memory")
+    auto rd = [&](int j, q35_u32x4 (&af)[4][2], q35_u32x4 (&bw)[4][2]) {
+        const unsigned so = (unsigned)((j % kRowsRing) * kRowsStage);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            Q35_WRD(af[s][0], aaddr[s] + so, 0);
+            Q35_WRD(af[s][1], aaddr[s] + so, 4096);
+            Q35_WRD(bw[s][0], baddr + so, s * 1024);
+            Q35_WRD(bw[s][1], baddr + so, B1 + s * 1024);
+        }
+    };
+#undef Q35_WRD
+    q35_f32x4 c[2][2], sum[2][2];
+    issue(0);
+    issue(1);
+    if (NS > 2) issue(2);
+    if (NS > 2) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");       // stage 0 landed
+    else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+    rd(0, fa[0], fb[0]);
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+        const int j = 2 * kb + jj, cur = jj;
+        // stage j + 1 landed for every wave (stage j + 2 may be in flight; none is issued past the
+        // last one) and stage j's fragments are in registers, so its slot takes stage j + 3; the
+        // vector-memory waits name no registers (see gemm_wide)
+        if (j + 2 < NS) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier"
+                     : "+v"(fa[cur][0][0]), "+v"(fa[cur][0][1]), "+v"(fa[cur][1][0]), "+v"(fa[cur][1][1]),
+                       "+v"(fa[cur][2][0]), "+v"(fa[cur][2][1]), "+v"(fa[cur][3][0]), "+v"(fa[cur][3][1]),
+                       "+v"(fb[cur][0][0]), "+v"(fb[cur][0][1]), "+v"(fb[cur][1][0]), "+v"(fb[cur][1][1]),
+                       "+v"(fb[cur][2][0]), "+v"(fb[cur][2][1]), "+v"(fb[cur][3][0]), "+v"(fb[cur][3][1])
+                     :: "memory");
+        if (j + 3 < NS) issue(j + 3);
+        if (j + 1 < NS) rd(j + 1, fa[cur ^ 1], fb[cur ^ 1]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int jn = 0; jn < 2; ++jn)
+                    c[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf(fa[cur][u][i]), as_bf(fb[cur][u][jn]),
+                                                                        jj == 0 && u == 0 ? (q35_f32x4){0.f, 0.f, 0.f, 0.f} : c[i][jn], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (jj == 1) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int jn = 0; jn < 2; ++jn)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sum[i][jn][r] = kb == 0 ? c[i][jn][r] : sum[i][jn][r] + c[i][jn][r];
+        }
     }
-    uint16_t* ob = wl + (size_t)wv * 1024;                           // [32 rows][32 cols]
+    __syncthreads();                   // the ring is drained by every wave: wave-private staging
+    store_wide64<EM>(a, sum, rb * 64 + wm * 32, nblk, (uint16_t*)dyn_lds, wv, lane);
+}
+
+// Few output tiles and a long K (N = 1024, K = 2048 / 3584 at some hundred rows: 64 x 64 blocks
+// fill a quarter of the CUs and walk K in dependent steps): 32 x 32 blocks whose 8 waves take the
+// k-blocks w, w + 8, ... each, so all of a block's operands are requested at once and the
+// k-blocks' chains meet in LDS, summed in k-block order. A wave's A slice (32 rows x 256 k) goes
+// through its own 16 KiB of LDS by DMA (in gemm_pre's layout: whole 128-byte lines per
+// instruction, XOR-swizzled for the fragment reads) and its weight fragments into registers; no
+// block barrier until the sum. K <= 4096: at most two k-blocks per wave. Bound by what a CU gets
+// from L2 (32 x 32 at K = 3584: 448 KiB a block, ~60 KiB per us): down_proj at 256 rows 9.0 us
+// against 28.1 in gemm_large_m's 64 blocks, at 32 rows (32 x 16 blocks) 5.9 against 25.5; out_proj
+// (K = 2048) at 256 rows 6.0 against 18.2.
+constexpr int kKsLds = 8 * 16384;
+
+template <int NT>
+__global__ void __launch_bounds__(512) gemm_ksplit(GemmArgs a) {
+    extern __shared__ q35_u32x4 dyn_lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int mb = (a.M + 31) / 32, ntiles = a.N / 16;
+    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+    const int nblk = (idx / mb) * 8 + xcd, rb = idx % mb;        // column blocks by XCD
+    if (nblk * NT >= ntiles) return;
+    const int KB = a.K >> 8;
+    const int row0 = rb * 32;
+    const int g = lane >> 4, r16 = lane & 15;
+    const int jrow = lane >> 3, jchunk = (lane & 7) ^ (lane >> 3);
+    char* mine = (char*)dyn_lds + wv * 16384;
+    // 16 KiB of A: KiB (mt, k-group gg, row half h), lane j = row * 8 + slot
+    const char* xb = (const char*)((const uint16_t*)a.X + (size_t)row0 * a.ldx);
+    unsigned xo[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int q = 0; q < 4; ++q)        // q = mt * 2 + h
+        xo[q] = (unsigned)(min(row0 + q * 8 + jrow, a.M - 1) - row0) * (unsigned)a.ldx * 2u + (unsigned)jchunk * 16u;
+    auto load_a = [&](int kb) {
 #pragma unroll
-        for (int jn = 0; jn < 2; ++jn)
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) ob[(i * 16 + 4 * (lane >> 4) + r) * 32 + jn * 16 + (lane & 15)] = f2bf(sum[i][jn][r]);
-    wave_sync();
+            for (int gg = 0; gg < 4; ++gg)
+                __builtin_amdgcn_global_load_lds((const void*)(uniform_ptr(xb + (size_t)kb * 512 + gg * 128) + xo[q]),
+                                                 (__attribute__((address_space(3))) void*)(mine + ((q >> 1) * 8 + gg * 2 + (q & 1)) * 1024), 16, 0, 0);
+    };
+    auto load_w = [&](int kb, q35_bf16x8 (&w)[NT][8]) {
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        const int ch = lane + 64 * q, row = ch >> 2, piece = ch & 3;
-        const int nt = nblk * 8 + wn * 2 + (piece >> 1), grow = row0 + row;
-        if (grow < a.M && nt < ntiles)
-            *(q35_u32x4*)(a.Y + (size_t)grow * a.ldy + nt * 16 + (piece & 1) * 8) = *(const q35_u32x4*)(ob + row * 32 + piece * 8);
+        for (int t = 0; t < NT; ++t) {
+            const int nt = min(nblk * NT + t, ntiles - 1);
+            const q35_bf16x8* wp = (const q35_bf16x8*)(a.W + ((size_t)nt * KB + kb) * 4096) + lane;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) w[t][s] = wp[s * 64];
+        }
+    };
+    auto chain = [&](const q35_bf16x8 (&w)[NT][8], q35_f32x4 (&c)[2][NT]) {
+        q35_u32x4 af[2][8];
+        const int h = r16 >> 3, rl = r16 & 7;
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                af[mt][s] = *(const q35_u32x4*)(mine + (mt * 8 + g * 2 + h) * 1024 + rl * 128 + ((s ^ rl) * 16));
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                c[mt][t] = (q35_f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < 8; ++s) c[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf(af[mt][s]), w[t][s], c[mt][t], 0, 0, 0);
+            }
+    };
+    q35_bf16x8 w0[NT][8], w1[NT][8];
+    q35_f32x4 c0[2][NT], c1[2][NT];
+    const bool two = wv + 8 < KB;
+    if (wv < KB) {
+        load_a(wv);
+        load_w(wv, w0);
+        if (two) load_w(wv + 8, w1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        chain(w0, c0);
+        if (two) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slice is in registers
+            load_a(wv + 8);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            chain(w1, c1);
+        }
+    }
+    // the chains through the waves' own regions (their slices are consumed): [tile][r][lane]
+    float* cw = (float*)mine;
+    if (wv < KB) {
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    cw[((mt * NT + t) * 4 + r) * 64 + lane] = c0[mt][t][r];
+                    if (two) cw[(8 * NT + (mt * NT + t) * 4 + r) * 64 + lane] = c1[mt][t][r];
+                }
+    }
+    __syncthreads();
+    // 2 NT tiles x 4 x 64 outputs over 512 threads, each summed in k-block order
+    const float* ca = (const float*)dyn_lds;
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+        const int e = q * 512 + tid, tl = e >> 8, r = (e >> 6) & 3, ln = e & 63;
+        float sum = ca[e];
+        for (int kb = 1; kb < KB; ++kb) sum = sum + ca[(kb & 7) * 4096 + (kb >> 3) * (8 * NT * 64) + e];
+        const int mt = tl / NT, t = tl % NT;
+        const int row = row0 + mt * 16 + 4 * (ln >> 4) + r, nt = nblk * NT + t;
+        if (row < a.M && nt < ntiles) a.Y[(size_t)row * a.ldy + nt * 16 + (ln & 15)] = f2bf(sum);
     }
 }
 
@@ -1408,9 +1651,44 @@ static hipError_t launch_wide(const GemmArgs& a, int em, hipStream_t st) {
     return hipGetLastError();
 }
 
+// The row-major forms read A and store Y in 16-byte pieces, with 32-bit offsets inside a block's rows
+static bool rows_ok(const GemmArgs& a) {
+    return a.ldx % 8 == 0 && a.ldy % 8 == 0 && (unsigned)a.ldx <= 1u << 24 &&
+           (((uintptr_t)a.X | (uintptr_t)a.Y | (uintptr_t)a.W) & 15) == 0;
+}
+
+template <int EM>
+static void launch_rows64(const GemmArgs& a, hipStream_t st) {
+    const int ncb = EM == kESiluMul ? (a.N / 32 + 3) / 4 : (a.N / 16 + 7) / 8, mb = (a.M + 63) / 64;
+    const int grid = ncb <= 8 ? ncb * ((mb + 7) / 8 * 8) : (ncb + 7) / 8 * 8 * mb;
+    hipLaunchKernelGGL((gemm_rows64<EM>), dim3(grid), dim3(512), kRowsLds, st, a);
+}
+template <int NT>
+static void launch_ksplit(const GemmArgs& a, hipStream_t st) {
+    const int nb = (a.N / 16 + NT - 1) / NT, mb = (a.M + 31) / 32;
+    hipLaunchKernelGGL((gemm_ksplit<NT>), dim3((nb + 7) / 8 * 8 * mb), dim3(512), kKsLds, st, a);
+}
+
+// Stored outputs of a plain A, K other than 1024 (down_proj, out_proj, o_proj, fc: N = 1024, K =
+// 2048 / 3584). 32 x 16 blocks of gemm_ksplit while one round of CUs (256) holds them, 32 x 32
+// while two rounds do, then gemm_rows64's 64 x 128 blocks. us at N = 1024, K = 3584 for rows 32 /
+// 128 / 256 / 512 / 768 / 1,999: 32 x 16 5.9 / 6.8 / 11.9 / 23.5 / 46.5 / 131, 32 x 32 7.7 / 8.8 /
+// 9.0 / 17.6 / 31.3 / 84.7, 64 x 128 20.7 / 21.3 / 21.4 / 21.8 / 21.9 / 24.8; the 64 x 64 blocks of
+// gemm_large_m took 25.5 / 28.1 / 28.1 / 28.2 / 28.3 / 35.1 (the same order at K = 2048).
+static void launch_longk(const GemmArgs& a, hipStream_t st) {
+    const long long mb = (a.M + 31) / 32;
+    if (mb * (a.N / 16) <= 256) launch_ksplit<1>(a, st);
+    else if (mb * ((a.N / 16 + 1) / 2) <= 512) launch_ksplit<2>(a, st);
+    else launch_rows64<kEStore>(a, st);
+}
+
 template <int EM>
 static void launch_large(const GemmArgs& a, hipStream_t st) {
     const int KB = a.K / 256;
+    if (EM == kEStore && a.K != kHidden && rows_ok(a)) {
+        launch_longk(a, st);
+        return;
+    }
     const int gz = EM == kEPartial ? (a.M >= a.forms.partial_rows ? 1 : KB) : 1;
     // 64-row tiles: more blocks in flight (W tiles are re-read from L2 by the M tiles)
     const int nb = EM == kESiluMul ? (a.N / 32 + 1) / 2 : (a.N / 16 + 3) / 4, mb = (a.M + 63) / 64;
@@ -1540,7 +1818,10 @@ hipError_t gemm_init() {
         hipFuncSetAttribute((const void*)gemm_wide<kESiluMul>, hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds) != hipSuccess ||
         hipFuncSetAttribute((const void*)gemm_wide64<kEStore>, hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds) != hipSuccess ||
         hipFuncSetAttribute((const void*)gemm_wide64<kESiluMul>, hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds) != hipSuccess ||
-        hipFuncSetAttribute((const void*)gemm_wide64<kEPartial>, hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds) != hipSuccess)
+        hipFuncSetAttribute((const void*)gemm_wide64<kEPartial>, hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds) != hipSuccess ||
+        hipFuncSetAttribute((const void*)gemm_rows64<kEStore>, hipFuncAttributeMaxDynamicSharedMemorySize, kRowsLds) != hipSuccess ||
+        hipFuncSetAttribute((const void*)gemm_ksplit<1>, hipFuncAttributeMaxDynamicSharedMemorySize, kKsLds) != hipSuccess ||
+        hipFuncSetAttribute((const void*)gemm_ksplit<2>, hipFuncAttributeMaxDynamicSharedMemorySize, kKsLds) != hipSuccess)
         return hipGetLastError();
     return hipSuccess;
 }
