@@ -26,7 +26,8 @@
 //                  cannot take);
 //                  a non-plain producer runs first as its own elementwise kernel
 //   gemm_ksplit    stored outputs, K != 1024, few tiles: 32-row blocks whose waves split K
-//   gemm_rows64    stored outputs from row-major A, more tiles: 64 x 128 blocks, an LDS ring
+//   gemm_rows64    row-major A, more tiles: 64 x 128 blocks, an LDS ring (also K = 1024 where its
+//                  rounds of blocks are well filled)
 // kEPartial (N = 1024 outputs feeding the residual add): each block computes ONE k-block
 // chain and stores it to kpart[kb][M][N]; the following add+norm kernel sums the chains in
 // k-block order. That keeps ~KB x more blocks in flight without cross-block atomics.
@@ -1722,6 +1723,20 @@ static void launch_large(const GemmArgs& a, hipStream_t st) {
         hipLaunchKernelGGL((gemm_large_m<EM, 4, 16>), dim3((nb16 + 7) / 8 * 8 * mb, 1, gz), dim3(1024), 0, st, a);
         return;
     }
+    if ((EM == kEStore || EM == kESiluMul) && a.K == kHidden && a.forms.gemm_pre == 1 && rows_ok(a)) {
+        // 64 x 128 blocks of gemm_rows64 (8.9 us the first round of 256, 7.8 each further one)
+        // unless gemm_pre's smaller blocks, which cost 3.3 us and 8.9 per 256 of those blocks, lose
+        // less in the last round: above (9 rounds - 3) / 10 of 256 blocks. us, gemm_pre -> rows64:
+        // gate|up with SwiGLU at 128 / 256 / 512 / 1,999 rows 8.3 / 12.7 / 22.0 / 79.5 -> 9.1 / 9.7 /
+        // 17.9 / 62.0 (112, 224, 448, 1,792 blocks); qkv (N = 5120) at 256 / 512 / 768 rows 9.6 /
+        // 14.5 / 20.6 -> 8.9 / 16.5 / 17.4 (160, 320, 480); in_proj (8224) at 256 / 384 13.4 / 17.5
+        // -> 15.9 / 16.7 (260, 390)
+        const long long b = (long long)(EM == kESiluMul ? (a.N / 32 + 3) / 4 : (a.N / 16 + 7) / 8) * mb;
+        if (10 * b > 256 * (9 * ((b + 255) / 256) - 3)) {
+            launch_rows64<EM == kESiluMul ? kESiluMul : kEStore>(a, st);
+            return;
+        }
+    }
     if ((EM == kEStore || EM == kESiluMul) && a.K == kHidden && a.forms.gemm_pre) {
         // 32-row blocks (64 KiB of A fragments: two blocks per CU); 64-row blocks (128 KiB,
         // one per CU) measured 10-35 % slower
@@ -1820,6 +1835,7 @@ hipError_t gemm_init() {
         hipFuncSetAttribute((const void*)gemm_wide64<kESiluMul>, hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds) != hipSuccess ||
         hipFuncSetAttribute((const void*)gemm_wide64<kEPartial>, hipFuncAttributeMaxDynamicSharedMemorySize, kWideLds) != hipSuccess ||
         hipFuncSetAttribute((const void*)gemm_rows64<kEStore>, hipFuncAttributeMaxDynamicSharedMemorySize, kRowsLds) != hipSuccess ||
+        hipFuncSetAttribute((const void*)gemm_rows64<kESiluMul>, hipFuncAttributeMaxDynamicSharedMemorySize, kRowsLds) != hipSuccess ||
         hipFuncSetAttribute((const void*)gemm_ksplit<1>, hipFuncAttributeMaxDynamicSharedMemorySize, kKsLds) != hipSuccess ||
         hipFuncSetAttribute((const void*)gemm_ksplit<2>, hipFuncAttributeMaxDynamicSharedMemorySize, kKsLds) != hipSuccess)
         return hipGetLastError();
