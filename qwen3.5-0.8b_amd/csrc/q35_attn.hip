@@ -173,14 +173,14 @@ __device__ __forceinline__ void score_slice(const AttnArgs& a, int lrow, int j, 
     for (int st = 0; st < 4; ++st)
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) m = fmaxf(m, sv[st][rr]);
-    m = fmaxf(m, __shfl_xor(m, 16, 64));
+    m = fmaxf(m, xor16(m));
     m = fmaxf(m, xor32(m));
     float e = 0.f;
 #pragma unroll
     for (int st = 0; st < 4; ++st)
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) e += sv[st][rr] > -INFINITY ? expf(sv[st][rr] - m) : 0.f;
-    e += __shfl_xor(e, 16, 64);
+    e += xor16(e);
     e += xor32(e);
     if (lane < 4 && t0 <= slot) {
         float* sp = stats + lane * stats_stride + 2 * q;
@@ -325,12 +325,10 @@ __device__ __forceinline__ void softmax_ml(const float* stats, size_t stats_stri
     const float* st = stats + h * stats_stride;
     float m = -INFINITY;
     for (int i = lane; i < nsl; i += 64) m = fmaxf(m, st[2 * i]);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    m = wave_max(m);
     float l = 0.f;
     for (int i = lane; i < nsl; i += 64) l += st[2 * i + 1] * expf(st[2 * i] - m);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o, 64);
+    l = wave_sum(l);
     if (lane == 0) {
         ml[h][0] = m;
         ml[h][1] = l;
@@ -442,9 +440,7 @@ __device__ __forceinline__ void wave_ml(const float* stats, size_t sst, int nsl,
         for (int h = 0; h < 4; ++h) m[h] = fmaxf(m[h], stats[h * sst + 2 * i]);
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-        for (int h = 0; h < 4; ++h) m[h] = fmaxf(m[h], __shfl_xor(m[h], o, 64));
+    for (int h = 0; h < 4; ++h) m[h] = wave_max(m[h]);
 #pragma unroll
     for (int h = 0; h < 4; ++h) l[h] = 0.f;
 #pragma unroll
@@ -461,9 +457,7 @@ __device__ __forceinline__ void wave_ml(const float* stats, size_t sst, int nsl,
         for (int h = 0; h < 4; ++h) l[h] += se[h] * expf(sm[h] - m[h]);
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-        for (int h = 0; h < 4; ++h) l[h] += __shfl_xor(l[h], o, 64);
+    for (int h = 0; h < 4; ++h) l[h] = wave_sum(l[h]);
 }
 
 // attention output element: bf16(bf16(sum of parts) * bf16(sigmoid(gate)))
@@ -619,14 +613,14 @@ __global__ void __launch_bounds__(256) attn_scores4(AttnArgs a) {
     for (int st = 0; st < 4; ++st)
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) m = fmaxf(m, sv[st][rr]);
-    m = fmaxf(m, __shfl_xor(m, 16, 64));
+    m = fmaxf(m, xor16(m));
     m = fmaxf(m, xor32(m));
     float e = 0.f;
 #pragma unroll
     for (int st = 0; st < 4; ++st)
 #pragma unroll
         for (int rr = 0; rr < 4; ++rr) e += sv[st][rr] > -INFINITY ? expf(sv[st][rr] - m) : 0.f;
-    e += __shfl_xor(e, 16, 64);
+    e += xor16(e);
     e += xor32(e);
     if (lane < 4) {
         float* sp = a.stats + ((size_t)r * kNq + 4 * j + lane) * a.max_chunks * 8 + 2 * q;
@@ -914,14 +908,14 @@ __global__ void __launch_bounds__(64 * W) attn_rows(AttnArgs a) {
                 for (int st = 0; st < 4; ++st)
 #pragma unroll
                     for (int rr = 0; rr < 4; ++rr) m = fmaxf(m, sv[u][st][rr]);
-                m = fmaxf(m, __shfl_xor(m, 16, 64));
+                m = fmaxf(m, xor16(m));
                 m = fmaxf(m, xor32(m));
                 float e = 0.f;
 #pragma unroll
                 for (int st = 0; st < 4; ++st)
 #pragma unroll
                     for (int rr = 0; rr < 4; ++rr) e += sv[u][st][rr] > -INFINITY ? expf(sv[u][st][rr] - m) : 0.f;
-                e += __shfl_xor(e, 16, 64);
+                e += xor16(e);
                 e += xor32(e);
                 const int t = 2 * u + tr;
                 if (g == 0 && (n & 7) < 4 && t0 <= lslot[u]) {

@@ -112,25 +112,44 @@ __device__ __forceinline__ const char* uniform_ptr(const char* p) {
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + expf(-x)); }
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-template <typename T>
-__device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-// __shfl_xor(v, 32) without LDS: v_permlane32_swap exchanges the two 32-lane halves
-// (result [1] holds the upper half's values for lanes < 32, [0] the lower half's for lanes >= 32)
+// Cross-lane moves without LDS (a __shfl is a ds_bpermute: an LDS round trip of ~100 cycles, and a
+// reduction's six of them are a dependent chain; a DPP or permlane move is one VALU instruction).
+// lane i <- lane i ^ 32: v_permlane32_swap exchanges the two 32-lane halves (result [1] holds the
+// upper half's values for lanes < 32, [0] the lower half's for lanes >= 32); lane i ^ 16 likewise.
 __device__ __forceinline__ float xor32(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
 }
+__device__ __forceinline__ float xor16(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float((threadIdx.x & 16) ? r[0] : r[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
 // lane i <- lane i + 4 within its row of 16 (DPP row_shl:4; 0 for the last 4 lanes of a row)
-__device__ __forceinline__ float row_down4(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x104, 0xf, 0xf, false));
+__device__ __forceinline__ float row_down4(float v) { return dpp<0x104>(v); }
+// All 64 lanes' sum / max by the xor tree 32, 16, 8, 4, 2, 1: after the folds by 32 and 16 a lane's
+// value depends on its place in its row of 16 only, so a rotation by 8 within the row is the
+// partner i ^ 8, then one by 4 the partner i ^ 4, then quad swaps. a + b = b + a exactly, so the
+// sums are the bits of the same tree of shuffles.
+__device__ __forceinline__ float wave_sum(float v) {
+    v += xor32(v);
+    v += xor16(v);
+    v += dpp<0x128>(v);      // row_ror:8
+    v += dpp<0x124>(v);      // row_ror:4
+    v += dpp<0x4E>(v);       // quad_perm [2,3,0,1]
+    v += dpp<0xB1>(v);       // quad_perm [1,0,3,2]
+    return v;
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    v = fmaxf(v, xor32(v));
+    v = fmaxf(v, xor16(v));
+    v = fmaxf(v, dpp<0x128>(v));
+    v = fmaxf(v, dpp<0x124>(v));
+    v = fmaxf(v, dpp<0x4E>(v));
+    v = fmaxf(v, dpp<0xB1>(v));
     return v;
 }
 
