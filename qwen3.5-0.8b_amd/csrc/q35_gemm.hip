@@ -225,8 +225,9 @@ __global__ void __launch_bounds__(TPB > 1 ? 256 : 1024) gemm_small_m(GemmArgs a)
     } else if (a.M == 1) {
         // Batch 1: lane c < 32 produces chunk c (k-block elements c*8 .. +8) with the same
         // produce_a arithmetic and row factors as the cooperative form below; the fragments
-        // of the row-0 lanes (g, s) = chunk 8g + s are gathered with wave shuffles -- no LDS
-        // round trip, no block barrier.
+        // of the row-0 lanes (g, s) = chunk 8g + s are gathered through the wave's own LDS -- no
+        // block barrier.
+        __shared__ q35_u32x4 own[EM == kEPartial ? 1 : 16][32];
         const int c = lane & 31;
         const int k0 = kb * 256 + c * 8;
         q35_u32x4 mine;
@@ -326,13 +327,15 @@ __global__ void __launch_bounds__(TPB > 1 ? 256 : 1024) gemm_small_m(GemmArgs a)
         }
         if (AM == kANormX && a.hout && blockIdx.x == 0 && lane < 32)
             *(q35_u32x4*)(a.hout + k0) = mine;
+        // chunk 8 g + s of the wave's 32 to the fragment of step s, row 0 (the other rows are zero):
+        // one 16-byte LDS write and 8 broadcast reads per lane (as 32 shuffles: 797 against 781 us
+        // per one-lane decode step at ctx 4,096)
+        own[wv][lane & 31] = mine;
+        wave_sync();
         const bool row0 = (lane & 15) == 0;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
-            const int src = 8 * g + s;
-            q35_u32x4 f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) f[i] = (uint32_t)__shfl((int)mine[i], src, 64);
+            const q35_u32x4 f = own[wv][8 * g + s];
             af[s] = row0 ? f : (q35_u32x4){0u, 0u, 0u, 0u};
         }
     } else {
