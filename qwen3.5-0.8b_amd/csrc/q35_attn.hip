@@ -234,6 +234,49 @@ __global__ void __launch_bounds__(256) attn_prep(AttnArgs a) {
     }
 }
 
+// A wave's q head into the score operand's columns c (bf16 of q) and c + 4 (its low part). Columns 8 ..
+// 15 (of a second row) stay as they are: an MFMA output column depends on its own B column only.
+__device__ __forceinline__ void make_q_head(const AttnArgs& a, const uint16_t* src, int pos, uint16_t (*qb)[256], int c) {
+    const int lane = threadIdx.x & 63;
+    float o[4];
+    head_norm_rope_wave(a, src, a.q_norm, pos, o);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const int d = lane + 64 * w;
+        const uint16_t hi = f2bf(o[w]);
+        qb[c][d] = hi;
+        qb[4 + c][d] = f2bf(o[w] - bf2f(hi));
+    }
+}
+// A wave's new K row (into the cache and, for the fragments already loaded, knew) and V row.
+__device__ __forceinline__ void make_kv_row(const AttnArgs& a, const uint16_t* prow, int pos, int lrow, int j, int slot,
+                                            uint16_t* knew) {
+    const int lane = threadIdx.x & 63;
+    float o[4];
+    head_norm_rope_wave(a, prow + kAttnKOff + j * 256, a.k_norm, pos, o);
+    const size_t base = lrow * a.kv_lane + a.kv_layer_off + (size_t)j * a.cap * 256;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const int d = lane + 64 * w;
+        const uint16_t kb = f2bf(o[w]);
+        knew[d] = kb;
+        a.kc[base + kv_tiled_offset(slot, d)] = kb;
+        a.vc[base + kv_v8_offset(slot, d)] = prow[kAttnVOff + j * 256 + d];
+    }
+}
+// The new K row in place of the fragments of sub-tile st in the lanes that hold its row (selects: with
+// a branch around them the compiler indexes the fragments by st and moves them to scratch memory).
+__device__ __forceinline__ void patch_k(const uint16_t* knew, int st, int slot, q35_u32x4 (*kf)[8]) {
+    const int lane = threadIdx.x & 63;
+    const bool mine = (lane & 15) == (slot & 15);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const q35_u32x4 v = *(const q35_u32x4*)&knew[s * 32 + (lane >> 4) * 8];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) kf[t][s] = mine && t == st ? v : kf[t][s];
+    }
+}
+
 // The split path with one row per lane (batch-1 decode): attn_prep folded into the slice
 // score kernel. Every block makes its 4 q heads itself; the block whose slice holds the new
 // slot also makes the new K row, appends K and V to the cache and patches its own K fragments
@@ -249,46 +292,14 @@ __global__ void __launch_bounds__(64) attn_scores_prep(AttnArgs a) {
     q35_u32x4 qf[8], kf[4][8];
     load_k_slice(a, lrow, j, q, slot, kf);
     const uint16_t* pr = a.proj + (size_t)r * kAttnInRows;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        float o[4];
-        head_norm_rope_wave(a, pr + (4 * j + i) * 512, a.q_norm, pos, o);
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const int d = lane + 64 * w;
-            const uint16_t hi = f2bf(o[w]);
-            qb[i][d] = hi;
-            qb[4 + i][d] = f2bf(o[w] - bf2f(hi));
-            qb[8 + i][d] = 0;
-            qb[12 + i][d] = 0;
-        }
-    }
     const bool own = q == (slot >> 6);
-    if (own) {
-        float o[4];
-        head_norm_rope_wave(a, pr + kAttnKOff + j * 256, a.k_norm, pos, o);
-        const size_t base = lrow * a.kv_lane + a.kv_layer_off + (size_t)j * a.cap * 256;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const int d = lane + 64 * w;
-            const uint16_t kb = f2bf(o[w]);
-            knew[d] = kb;
-            a.kc[base + kv_tiled_offset(slot, d)] = kb;
-            a.vc[base + kv_v8_offset(slot, d)] = pr[kAttnVOff + j * 256 + d];
-        }
-    }
+    for (int i = 0; i < 4; ++i) make_q_head(a, pr + (4 * j + i) * 512, pos, qb, i);
+    if (own) make_kv_row(a, pr, pos, lrow, j, slot, knew);
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < 8; ++s) qf[s] = *(const q35_u32x4*)&qb[n][s * 32 + g * 8];
-    if (own && n == (slot & 15)) {
-        const int st = (slot >> 4) - q * 4;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            if (t == st) {
-#pragma unroll
-                for (int s = 0; s < 8; ++s) kf[t][s] = *(const q35_u32x4*)&knew[s * 32 + g * 8];
-            }
-    }
+    if (own) patch_k(knew, (slot >> 4) - q * 4, slot, kf);
     score_slice<false>(a, lrow, j, q, slot, qf, kf, 0, a.sc + ((size_t)r * kNq + 4 * j) * a.sc_ld, a.sc_ld,
                        a.stats + ((size_t)r * kNq + 4 * j) * a.max_chunks * 8, (size_t)a.max_chunks * 8);
 }
@@ -539,29 +550,8 @@ __global__ void __launch_bounds__(256) attn_scores4(AttnArgs a) {
     if (PREP) {
         const int pos = a.rm.pos[r];
         const uint16_t* pr = a.proj + (size_t)r * kAttnInRows;
-        float o[4];
-        head_norm_rope_wave(a, pr + (4 * j + wv) * 512, a.q_norm, pos, o);
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const int d = lane + 64 * w;
-            const uint16_t hi = f2bf(o[w]);
-            qb[wv][d] = hi;
-            qb[4 + wv][d] = f2bf(o[w] - bf2f(hi));
-            qb[8 + wv][d] = 0;
-            qb[12 + wv][d] = 0;
-        }
-        if (own && wv == 0) {
-            head_norm_rope_wave(a, pr + kAttnKOff + j * 256, a.k_norm, pos, o);
-            const size_t base = lrow * a.kv_lane + a.kv_layer_off + (size_t)j * a.cap * 256;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                const int d = lane + 64 * w;
-                const uint16_t kb = f2bf(o[w]);
-                knew[d] = kb;
-                a.kc[base + kv_tiled_offset(slot, d)] = kb;
-                a.vc[base + kv_v8_offset(slot, d)] = pr[kAttnVOff + j * 256 + d];
-            }
-        }
+        make_q_head(a, pr + (4 * j + wv) * 512, pos, qb, wv);
+        if (own && wv == 0) make_kv_row(a, pr, pos, lrow, j, slot, knew);
     } else {
         const float* qp = a.q + ((size_t)r * kNq + 4 * j + wv) * 256;
 #pragma unroll
@@ -679,7 +669,11 @@ __global__ void __launch_bounds__(64) attn_pv4(AttnArgs a) {
 // half idle in between); the halves of one block meet at every barrier, so both items end
 // together. A half with fewer parts runs idle parts (its loads clamped, its sums not added)
 // to keep the barrier count equal.
-template <bool NT, int NI>
+// PREP (one row per lane, no lane twice): the item's q heads and its new K / V row are made here, by
+// wave (q head wv; wave 0 also the K row, into the q staging's unused column 8), instead of by
+// attn_prep (8 us and a launch gap at 256 rows); the K fragments of the new slot, loaded before it
+// was written, are patched from there.
+template <bool NT, int NI, bool PREP>
 __global__ void __launch_bounds__(256 * NI) attn_fused(AttnArgs a, int lds_slots) {
     extern __shared__ float fl[];
     const int half = NI == 1 ? 0 : (int)(threadIdx.x >> 8);
@@ -716,11 +710,23 @@ __global__ void __launch_bounds__(256 * NI) attn_fused(AttnArgs a, int lds_slots
         const int wv = tid >> 6;
         q35_u32x4 kf[4][8];
         load_k_slice<NT>(a, lrow, j, wv, slot, kf);
-        load_q_frags(a, r, j, qb, qf);
+        if constexpr (PREP) {
+            const int lane = tid & 63, n = lane & 15, g = lane >> 4;
+            const uint16_t* prow = a.proj + (size_t)r * kAttnInRows;
+            const int pos = a.rm.pos[r];
+            make_q_head(a, prow + (4 * j + wv) * 512, pos, qb, wv);
+            if (wv == 0 && active) make_kv_row(a, prow, pos, lrow, j, slot, qb[8]);
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < 8; ++s) qf[s] = *(const q35_u32x4*)&qb[n][s * 32 + g * 8];
+        } else {
+            load_q_frags(a, r, j, qb, qf);
+        }
         // wave wv takes slices 4c + wv; the last one refills nothing (no loads past the end
         // ahead of the V stream's first loads)
         for (int c = 0; c + 1 < nch; ++c)
             score_slice<true, NT>(a, lrow, j, 4 * c + wv, slot, qf, kf, 4 * (c + 1) + wv, scl, lds_slots, stl, sst);
+        if (PREP && nch > 0 && (slot >> 6) == 4 * (nch - 1) + wv) patch_k(qb[8], (slot >> 4) & 3, slot, kf);
         if (nch > 0) score_slice<false, NT>(a, lrow, j, 4 * (nch - 1) + wv, slot, qf, kf, 0, scl, lds_slots, stl, sst);
     }
     if (NI > 1 && tid == 0) nparts_all[half] = nparts;
@@ -775,7 +781,9 @@ __global__ void __launch_bounds__(256 * NI) attn_fused(AttnArgs a, int lds_slots
 // what it wrote, after a block barrier.
 // W = 8 (engine option attn_rows 2): one block of 8 waves per CU -- the memory parallelism of
 // two 4-wave blocks, and three times the LDS tail; P.V then takes 2 dim tiles per wave.
-template <int T, int W = 4>
+// PREP (no lane twice): q and the T new K / V rows made here, one head per wave and turn, instead of
+// by attn_prep; the K fragments of the new slots are patched from LDS where they are used.
+template <int T, int W, bool PREP>
 __global__ void __launch_bounds__(64 * W) attn_rows(AttnArgs a) {
     extern __shared__ float stl_all[];                  // [T][4][8 * max_chunks] slice stats, then
                                                         // the LDS tail [T][4][lpn * 128]
@@ -799,6 +807,38 @@ __global__ void __launch_bounds__(64 * W) attn_rows(AttnArgs a) {
     const int p0 = max(slot / kPart + 1 - lpn, 0);     // first part in the LDS tail
     // q fragments: tile u, column 8 (t % 2) + h = bf16(q) of row t = 2u + t % 2, head h, and
     // + 4 its low part (zero columns for a missing row), as load_q_frags makes them
+    // the new K rows, in the columns of q tile 1 that no row has
+    uint16_t(*knew)[256] = &qbuf[1][8];
+    q35_u32x4 kf[2][8];
+    const int nch = (slot / 64 + W) / W;                 // rounds of W slices
+    // K two sub-tiles ahead (kf[st % 2] holds sub-tile st; the registers of sub-tile st are refilled
+    // with sub-tile st + 2, then the next slice's); the first slice's sub-tile 0 strictly before its
+    // sub-tile 1: the loop head's wait for sub-tile 0 must hold on entry too, and with sub-tile 0
+    // loaded last it would drain the whole prefetch (and the previous slice's score stores) at
+    // every slice
+    load_k_sub<true>(a, lrow, j, W * (nch - 1) + wv, 0, slot, kf[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_k_sub<true>(a, lrow, j, W * (nch - 1) + wv, 1, slot, kf[1]);
+    if constexpr (PREP) {
+        // heads 0 .. 4T-1: q of (row, head); 4T .. 5T-1: the new K row of row i - 4T
+        for (int i = __builtin_amdgcn_readfirstlane(wv); i < 5 * T; i += W) {
+            const int t = i < 4 * T ? i >> 2 : i - 4 * T;
+            const uint16_t* prow = a.proj + (size_t)(r0 + t) * kAttnInRows;
+            const int pos = a.rm.pos[r0 + t];
+            if (i >= 4 * T) {
+                make_kv_row(a, prow, pos, lrow, j, a.rm.slot[r0 + t], knew[t]);
+                continue;
+            }
+            float o[4];
+            head_norm_rope_wave(a, prow + (4 * j + (i & 3)) * 512, a.q_norm, pos, o);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const uint16_t hi = f2bf(o[w]);
+                qbuf[t >> 1][8 * (t & 1) + (i & 3)][lane + 64 * w] = hi;
+                qbuf[t >> 1][8 * (t & 1) + (i & 3) + 4][lane + 64 * w] = f2bf(o[w] - bf2f(hi));
+            }
+        }
+    } else
     if (tid < 256) {
 #pragma unroll
         for (int t = 0; t < 2 * NU; ++t)
@@ -817,23 +857,16 @@ __global__ void __launch_bounds__(64 * W) attn_rows(AttnArgs a) {
             }
     }
     __syncthreads();
+    int smin = slot_t[0];
+#pragma unroll
+    for (int t = 1; t < T; ++t) smin = min(smin, slot_t[t]);
     // scores: wave wv takes slices W c + wv (score_slice's arithmetic, one MFMA chain per tile)
     {
-        // q fragments in registers, K two sub-tiles ahead (kf[st % 2] holds sub-tile st; the
-        // registers of sub-tile st are refilled with sub-tile st + 2, then the next slice's)
         q35_u32x4 qf[NU][8];
 #pragma unroll
         for (int u = 0; u < NU; ++u)
 #pragma unroll
             for (int s = 0; s < 8; ++s) qf[u][s] = *(const q35_u32x4*)&qbuf[u][n][s * 32 + g * 8];
-        q35_u32x4 kf[2][8];
-        // the first slice's sub-tile 0 strictly before its sub-tile 1: the loop head's wait for
-        // sub-tile 0 must hold on entry too, and with sub-tile 0 loaded last it would drain the
-        // whole prefetch (and the previous slice's score stores) at every slice
-        const int nch = (slot / 64 + W) / W;             // rounds of W slices
-        load_k_sub<true>(a, lrow, j, W * (nch - 1) + wv, 0, slot, kf[0]);
-        __builtin_amdgcn_sched_barrier(0);
-        load_k_sub<true>(a, lrow, j, W * (nch - 1) + wv, 1, slot, kf[1]);
         // this block's rows of the score scratch as a buffer resource (byte offsets)
         const __amdgpu_buffer_rsrc_t scres = __builtin_amdgcn_make_buffer_rsrc(
             (void*)uniform_ptr((const char*)(a.sc + (size_t)r0 * kNq * a.sc_ld)), 0, T * kNq * a.sc_ld * 4, 0x00020000);
@@ -853,6 +886,14 @@ __global__ void __launch_bounds__(64 * W) attn_rows(AttnArgs a) {
             float sv[NU][4][4];
 #pragma unroll
             for (int st = 0; st < 4; ++st) {
+                if (PREP && 4 * q + st >= smin >> 4) {   // new K rows: their loads may be stale
+#pragma unroll
+                    for (int t = 0; t < T; ++t)
+                        if (slot_t[t] >> 4 == 4 * q + st && n == (slot_t[t] & 15)) {
+#pragma unroll
+                            for (int s = 0; s < 8; ++s) kf[st & 1][s] = *(const q35_u32x4*)&knew[t][s * 32 + g * 8];
+                        }
+                }
                 q35_f32x4 acc[NU];
 #pragma unroll
                 for (int u = 0; u < NU; ++u) {
@@ -1258,16 +1299,16 @@ __global__ void __launch_bounds__(256) attn_prompt(AttnArgs a) {
 }
 
 hipError_t attn_init() {
-    hipError_t e = hipFuncSetAttribute((const void*)attn_fused<true, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)attn_fused<false, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)attn_fused<true, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, kFused2MaxLds);
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)attn_rows<2, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, kRowsLdsDyn8);
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)attn_rows<3, 8>, hipFuncAttributeMaxDynamicSharedMemorySize, kRowsLdsDyn8);
-    if (e != hipSuccess) return e;
+    const struct { const void* f; int lds; } big[] = {
+        {(const void*)attn_fused<true, 1, true>, 96 * 1024}, {(const void*)attn_fused<true, 1, false>, 96 * 1024},
+        {(const void*)attn_fused<false, 1, false>, 96 * 1024},
+        {(const void*)attn_fused<true, 2, true>, kFused2MaxLds}, {(const void*)attn_fused<true, 2, false>, kFused2MaxLds},
+        {(const void*)attn_rows<2, 8, true>, kRowsLdsDyn8}, {(const void*)attn_rows<2, 8, false>, kRowsLdsDyn8},
+        {(const void*)attn_rows<3, 8, true>, kRowsLdsDyn8}, {(const void*)attn_rows<3, 8, false>, kRowsLdsDyn8}};
+    for (const auto& b : big) {
+        const hipError_t e = hipFuncSetAttribute(b.f, hipFuncAttributeMaxDynamicSharedMemorySize, b.lds);
+        if (e != hipSuccess) return e;
+    }
     return hipFuncSetAttribute((const void*)attn_prompt, hipFuncAttributeMaxDynamicSharedMemorySize, kPrLds);
 }
 
@@ -1285,8 +1326,6 @@ static bool use_fused2(const AttnArgs& a) {
     if (a.force == kAttnFused) return false;
     return a.T == 1 && (a.fused_pair || a.force == kAttnFusedPair) && 2 * fused_lds(a) <= (size_t)kFused2MaxLds;
 }
-// one row per lane on the split path: the prep runs inside the slice score kernel
-static bool prep_in_scores(const AttnArgs& a) { return !use_fused(a) && a.T == 1; }
 // a lane's 2-3 verify rows in one block when the (lane, kv head) blocks fill the CUs
 static int rows_w(const AttnArgs& a) { return a.rows_form == 2 ? 8 : 4; }
 static bool use_rows(const AttnArgs& a) {
@@ -1304,6 +1343,21 @@ static bool use_prompt(const AttnArgs& a) {
     return a.prompt_flash && shape;
 }
 
+// The form makes q and the new K / V rows itself: the split path with one row per lane; the fused
+// form with one row per lane and the rows form, whose blocks read only rows they make, as long as
+// no lane occurs twice (another row's block would append to the same lane). The fused form up to
+// 600,000 slots in all: there the launch it saves is 2 .. 8 % (us, attn_prep -> folded: 256 lanes x
+// 1,000 slots 117.4 -> 113.9, 130 x 4,000 223 -> 212); beyond it a full chip streaming at the HBM
+// rate pays more for every block's appended rows at once (224 x 3,000 237 -> 242, 240 x 4,000 323
+// -> 350). The rows form gains everywhere (250 lanes x 3 rows x 2,000: 200 -> 198, ragged 158 -> 151).
+static bool prep_folded(const AttnArgs& a) {
+    if (use_prompt(a)) return false;
+    if (use_rows(a)) return a.distinct;
+    return a.T == 1 && (!use_fused(a) || (a.distinct && (long long)a.R * a.cap <= 600000));
+}
+// the split path's part of that
+static bool prep_in_scores(const AttnArgs& a) { return a.T == 1; }
+
 bool attn_prompt_form(const AttnArgs& a) { return use_prompt(a); }
 
 // Whether the forced form can run this shape (kAttnAuto always can).
@@ -1320,7 +1374,7 @@ bool attn_form_ok(const AttnArgs& a) {
 
 hipError_t launch_attn_prep(const AttnArgs& a, hipStream_t st) {
     if (a.R <= 0 || a.max_chunks <= 0) return hipErrorInvalidValue;
-    if (prep_in_scores(a)) return hipSuccess;
+    if (prep_folded(a)) return hipSuccess;
     hipLaunchKernelGGL(attn_prep, dim3((a.R * (kNq + kNkv) + 3) / 4), dim3(256), 0, st, a);
     return hipGetLastError();
 }
@@ -1337,22 +1391,29 @@ hipError_t launch_attn_core(const AttnArgs& a, hipStream_t st) {
     } else if (use_rows(a)) {
         const int W = rows_w(a);
         const size_t lds = rows_lds_bytes(a.T, a.max_chunks, W);
-        if (W == 8) {
-            if (a.T == 2) hipLaunchKernelGGL((attn_rows<2, 8>), dim3(a.R / 2 * kNkv), dim3(512), lds, st, a);
-            else hipLaunchKernelGGL((attn_rows<3, 8>), dim3(a.R / 3 * kNkv), dim3(512), lds, st, a);
-        } else if (a.T == 2) hipLaunchKernelGGL((attn_rows<2, 4>), dim3(a.R / 2 * kNkv), dim3(256), lds, st, a);
-        else hipLaunchKernelGGL((attn_rows<3, 4>), dim3(a.R / 3 * kNkv), dim3(256), lds, st, a);
+#define Q35_ROWS(TV, WV)                                                                                          \
+    if (a.T == TV && W == WV) {                                                                                   \
+        if (prep_folded(a)) hipLaunchKernelGGL((attn_rows<TV, WV, true>), dim3(a.R / TV * kNkv), dim3(64 * WV), lds, st, a); \
+        else hipLaunchKernelGGL((attn_rows<TV, WV, false>), dim3(a.R / TV * kNkv), dim3(64 * WV), lds, st, a);     \
+    }
+        Q35_ROWS(2, 8) Q35_ROWS(3, 8) Q35_ROWS(2, 4) Q35_ROWS(3, 4)
+#undef Q35_ROWS
     } else if (use_fused(a)) {
         if (a.T < 1 || a.R % a.T) return hipErrorInvalidValue;
         const int pairs = a.R / a.T * kNkv;
         const int nseg = std::max(1, 8 / pairs), seg = (a.T + nseg - 1) / nseg;
         const dim3 grid((pairs * nseg + 7) / 8 * seg * 8);
-        if (use_fused2(a))
-            hipLaunchKernelGGL((attn_fused<true, 2>), dim3((grid.x + 15) / 16 * 8), dim3(512), 2 * lds, st, a, lds_slots);
-        else if (a.T == 1)
-            hipLaunchKernelGGL((attn_fused<true, 1>), grid, dim3(256), lds, st, a, lds_slots);
-        else
-            hipLaunchKernelGGL((attn_fused<false, 1>), grid, dim3(256), lds, st, a, lds_slots);
+        const bool prep = prep_folded(a);
+        if (use_fused2(a)) {
+            const dim3 g2((grid.x + 15) / 16 * 8);
+            if (prep) hipLaunchKernelGGL((attn_fused<true, 2, true>), g2, dim3(512), 2 * lds, st, a, lds_slots);
+            else hipLaunchKernelGGL((attn_fused<true, 2, false>), g2, dim3(512), 2 * lds, st, a, lds_slots);
+        } else if (a.T == 1) {
+            if (prep) hipLaunchKernelGGL((attn_fused<true, 1, true>), grid, dim3(256), lds, st, a, lds_slots);
+            else hipLaunchKernelGGL((attn_fused<true, 1, false>), grid, dim3(256), lds, st, a, lds_slots);
+        } else {
+            hipLaunchKernelGGL((attn_fused<false, 1, false>), grid, dim3(256), lds, st, a, lds_slots);
+        }
     } else {
         if (a.force == kAttnSplit4 || (a.force != kAttnSplit && a.split4)) {
             if (prep_in_scores(a))

@@ -181,6 +181,7 @@ struct AttnArgs {
     int out_tiled;         // attn_prompt only: out in the GEMMs' tiled fragment layout (K = 2048)
     int R;
     int T;                 // rows per lane (a lane's rows are consecutive; MTP verify: k + 1)
+    int distinct;          // no lane occurs twice: a block may make the q and K / V rows it reads itself
     const float* inv_freq; // [32] f32 rope inverse frequencies
     int prompt_flash;      // KernelForms::attn_prompt of the calling engine
     int split4;            // KernelForms::attn_split4: split path in 4-wave score / dim-split P.V blocks
