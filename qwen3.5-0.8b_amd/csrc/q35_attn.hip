@@ -1321,12 +1321,20 @@ static bool use_fused(const AttnArgs& a) {
     if (a.force != kAttnAuto) return false;
     return a.R >= 64 && fused_fits(a);
 }
-// two items per block (one row per lane) when both items' LDS fits the CU
+// Two items per block (one row per lane) when both items' LDS fits the CU and there are more items
+// than CUs: up to 256 of them run one per CU, where pairing would leave half of the CUs idle and
+// let the longer lane of a pair hold up the shorter one. us, one item -> two per block: 64 lanes x
+// 4,000 slots 127 -> 193, 128 x 1,000 67 -> 76, 128 x 500 .. 4,000 ragged 137 -> 192; beyond, 160 x
+// 4,000 263 -> 231, 160 x 1,000 88 -> 81. (Below 64 lanes the split path: 48 x 4,000 103, one item
+// per block 127; 48 x 1,000 49 and 55.)
 static bool use_fused2(const AttnArgs& a) {
-    if (a.force == kAttnFused) return false;
-    return a.T == 1 && (a.fused_pair || a.force == kAttnFusedPair) && 2 * fused_lds(a) <= (size_t)kFused2MaxLds;
+    if (a.force == kAttnFused || a.T != 1 || 2 * fused_lds(a) > (size_t)kFused2MaxLds) return false;
+    return a.force == kAttnFusedPair || (a.fused_pair && a.R * kNkv > 256);
 }
-// a lane's 2-3 verify rows in one block when the (lane, kv head) blocks fill the CUs
+// A lane's 2-3 verify rows in one block from 192 rows on: the K/V stream once instead of once per
+// row. us, one block per row -> rows form: 100 lanes x 2 x 3,000 171 -> 123, ragged 143 -> 101; 64 x 3
+// x 4,000 185 -> 145, ragged 138 -> 125; 64 x 3 x 1,000 58.6 -> 59.3, 64 x 2 x 4,000 125 -> 127, 32 x 3 x
+// 4,000 99 -> 124.
 static int rows_w(const AttnArgs& a) { return a.rows_form == 2 ? 8 : 4; }
 static bool use_rows(const AttnArgs& a) {
     // the slice stats (and the tail) fit the block's dynamic LDS
@@ -1334,7 +1342,7 @@ static bool use_rows(const AttnArgs& a) {
                        rows_lds_bytes(a.T, a.max_chunks, rows_w(a)) <= (rows_w(a) == 8 ? (size_t)kRowsLdsDyn8 : 65536);
     if (a.force == kAttnRows) return shape;
     if (a.force != kAttnAuto) return false;
-    return a.rows_form && shape && a.R / a.T * kNkv >= 256;
+    return a.rows_form && shape && a.R >= 192;
 }
 static bool use_prompt(const AttnArgs& a) {
     const bool shape = a.T >= 64 && a.R == a.T;

@@ -24,7 +24,7 @@ def rows_at(h, lane, p, T):
 
 
 @pytest.mark.parametrize("T", [1, 2, 3])
-@pytest.mark.parametrize("B", [2, 64, 130, 256])
+@pytest.mark.parametrize("B", [2, 63, 64, 96, 128, 129, 256])
 def test_folded_prep_equals_split(harness, B, T):
     h = harness
     rng = np.random.default_rng(B * 4 + T)
