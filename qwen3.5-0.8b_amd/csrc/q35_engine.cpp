@@ -1767,16 +1767,12 @@ static void op_gdn(q35_engine* e, const uint16_t* proj, const uint16_t* conv_w, 
     REQ(!y == !gnorm, Q35_ERR_ARG, "y and gnorm go together");
     REQ(!y || B <= e->R, Q35_ERR_CAP, "B exceeds max_rows (the norm staging is engine scratch)");
     // rows b = lanes b (T = 1); per lane two slots: 0 = input state, 1 = output state
-    std::vector<int> lanes(B);
-    for (int i = 0; i < B; ++i) lanes[i] = i;
-    int* dl = dalloc<int>(B);
-    copy_sync(e, dl, lanes.data(), B * sizeof(int), hipMemcpyHostToDevice);
     GdnArgs g{};
     g.proj = proj; g.o = o; g.conv_w = conv_w; g.A_log = A_log; g.dt_bias = dt_bias;
     g.S = S2; g.S_lane = 2 * kSLayer; g.S_slot = kSLayer; g.S_layer = 0;
     g.win = W2; g.W_lane = 2 * kWLayer; g.W_slot = kWLayer; g.W_layer = 0;
     g.cur = nullptr; g.nslots = 2; g.ckpt = 0;
-    g.lane = dl; g.T = 1; g.nlanes = B;
+    g.lane = nullptr; g.T = 1; g.nlanes = B;       // row b is lane b
     const int cs = B <= 8 ? 8 : B <= 32 ? 4 : B <= 64 ? 2 : 1;
     const bool whole = cs == 1 || form == 1;           // whole-head blocks: norm in the epilogue
     if (whole && y) { g.y = y; g.gnorm = gnorm; }
@@ -1790,7 +1786,6 @@ static void op_gdn(q35_engine* e, const uint16_t* proj, const uint16_t* conv_w, 
         HCK(launch_produce(a, kAGatedNorm, e->st));
     }
     HCK(hipStreamSynchronize(e->st));
-    HCK(hipFree(dl));
 }
 
 int q35_op_gdn_step(q35_engine* e, const uint16_t* proj, const uint16_t* conv_w, const uint16_t* A_log,
@@ -1887,8 +1882,16 @@ int q35_op_attn_decode(q35_engine* e, q35_state* s, int layer, const int32_t* la
                 e->h_tok[r] = 0; e->h_lane[r] = l; e->h_pos[r] = p + t; e->h_slot[r] = p + t;
             }
         }
-        stage_rcur(e, s, R);
-        upload_rows(e, R);
+        // lanes and positions are all the attention kernels read of the row metadata
+        if (n <= kRowArgs && s->lanes <= 65536) {
+            RowArgs ra;
+            for (int i = 0; i < n; ++i) { ra.lane[i] = (uint16_t)e->h_lane[i * T]; ra.pos[i] = e->h_pos[i * T]; }
+            ++e->meta_epoch;
+            HCK(launch_set_rows(ra, n, T, e->rlane, e->rpos, e->rslot, e->st));
+        } else {
+            stage_rcur(e, s, R);
+            upload_rows(e, R);
+        }
         AttnArgs a{};
         a.proj = proj; a.q_norm = q_norm; a.k_norm = k_norm;
         a.kc = s->kc; a.vc = s->vc; a.kv_lane = s->kv_lane(); a.kv_layer_off = (long long)layer * 2 * s->capT * 256;

@@ -63,7 +63,7 @@ __global__ void __launch_bounds__(256) gdn_kernel(GdnArgs a) {
     const uint2 cpk = *(const uint2*)(a.conv_w + (size_t)cqk * 4);
     const uint2 dpk = *(const uint2*)(a.conv_w + (size_t)cvc * 4);
     const uint16_t alogr = a.A_log[h], dtbr = a.dt_bias[h];
-    const int lane = a.lane[gi * a.T];
+    const int lane = a.lane ? a.lane[gi * a.T] : gi;
     const int cur = a.cur ? a.cur[gi * a.T] : 0;
     const int wcur = a.wcur ? a.wcur[gi * a.T] : cur;
     const int pnd = a.pend ? a.pend[gi * a.T] : 0;
@@ -351,7 +351,7 @@ __global__ void __launch_bounds__(256, 2) gdn_persist(GdnArgs a, int nitems) {
     const int nk = (nitems - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
     for (int k = tid; k < nk; k += 256) {
         const int gi = (((int)blockIdx.x + k * (int)gridDim.x) >> 4) * TR;   // the lane's first row
-        const int ln = a.lane[gi];
+        const int ln = a.lane ? a.lane[gi] : gi / TR;
         const int cu = a.cur ? a.cur[gi] : 0;
         const int wc = a.wcur ? a.wcur[gi] : cu;
         const int pn = a.pend ? a.pend[gi] : 0;

@@ -158,4 +158,17 @@ hipError_t launch_mtp_concat(const int* tok, const uint16_t* E, const uint16_t* 
     return hipGetLastError();
 }
 
+// The arguments are indexed by thread: read from the argument segment in memory, a few lines.
+__global__ void __launch_bounds__(256) set_rows_kernel(RowArgs a, int n, int T, int* lane, int* pos, int* slot) {
+    const int r = blockIdx.x * 256 + threadIdx.x, i = r / T;
+    if (i >= n) return;
+    lane[r] = a.lane[i];
+    pos[r] = slot[r] = a.pos[i] + r % T;
+}
+hipError_t launch_set_rows(const RowArgs& a, int n, int T, int* lane, int* pos, int* slot, hipStream_t st) {
+    if (n <= 0 || n > kRowArgs || T <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(set_rows_kernel, dim3((n * T + 255) / 256), dim3(256), 0, st, a, n, T, lane, pos, slot);
+    return hipGetLastError();
+}
+
 }  // namespace q35

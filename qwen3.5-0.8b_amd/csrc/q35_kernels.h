@@ -129,7 +129,7 @@ struct GdnArgs {
     int defer;                 // decode rows (T = 1, ckpt = 0): a lane with n < defer pending rows
                                // records this row as pending row n of its own set (factors) and
                                // keeps slot cur; otherwise its state goes to slot (cur + 1) % nslots
-    const int* lane;           // [R] state lane of each row
+    const int* lane;           // [R] state lane of each row (null: row group i is lane i)
     int T;                     // rows per lane (rows of one lane are consecutive)
     int nlanes;
     // Optional fused gated RMSNorm (whole-head blocks and the chunked form's output kernel):
@@ -208,6 +208,11 @@ hipError_t launch_gen_normal_plain(uint64_t key, float scale, long long n, uint1
 hipError_t launch_gen_normal_f32(uint64_t key, float scale, long long n, float* dst,
                                  hipStream_t st);
 
+// Row metadata of n lanes x T rows from kernel arguments (a short call's lanes and positions need no
+// host-to-device copy): row i * T + t gets lane[i], position and cache slot pos[i] + t.
+constexpr int kRowArgs = 256;
+struct RowArgs { int pos[kRowArgs]; uint16_t lane[kRowArgs]; };
+hipError_t launch_set_rows(const RowArgs& a, int n, int T, int* lane, int* pos, int* slot, hipStream_t st);
 hipError_t launch_tile(const uint16_t* src, int N, int K, uint16_t* dst, int row_off, int inverse,
                        hipStream_t st);
 hipError_t launch_copy_rows(const uint16_t* src, const int* src_rows, uint16_t* dst, const int* dst_rows,
