@@ -14,7 +14,8 @@
 //   attn_pv     (row, kv head, 128-slot part) global (max, sum) from the chunk stats,
 //               p = bf16(e/l), partial P.V per part on MFMA (V cache in 8-slot groups)
 //   attn_combine (row, q head)      sum of the parts in order, bf16, times bf16(sigmoid(gate))
-// plus attn_rows (MTP verify: a lane's rows in one block) and attn_prompt (prompt waves).
+// plus attn_rows and attn_seg_* (MTP verify: a lane's rows in one block, or in one block per segment)
+// and attn_prompt (prompt waves).
 // The k cache holds bf16(k post-rope); the reference's torch path keeps it in f32, so
 // k's rotated dims carry one extra bf16 rounding here (the cache layout is bf16 by design).
 #include <algorithm>
@@ -225,12 +226,15 @@ __global__ void __launch_bounds__(256) attn_prep(AttnArgs a) {
     }
     const int j = hh - kNq, slot = a.rm.slot[r];
     const size_t base = a.rm.lane[r] * a.kv_lane + a.kv_layer_off + (size_t)j * a.cap * 256;
+    uint16_t v[4];                          // before the K stores (see make_kv_row)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) v[w] = pr[kAttnVOff + j * 256 + lane + 64 * w];
     head_norm_rope_wave(a, pr + kAttnKOff + j * 256, a.k_norm, pos, o);
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         const int d = lane + 64 * w;
         a.kc[base + kv_tiled_offset(slot, d)] = f2bf(o[w]);
-        a.vc[base + kv_v8_offset(slot, d)] = pr[kAttnVOff + j * 256 + d];
+        a.vc[base + kv_v8_offset(slot, d)] = v[w];
     }
 }
 
@@ -248,10 +252,14 @@ __device__ __forceinline__ void make_q_head(const AttnArgs& a, const uint16_t* s
         qb[4 + c][d] = f2bf(o[w] - bf2f(hi));
     }
 }
-// A wave's new K row (into the cache and, for the fragments already loaded, knew) and V row.
+// A wave's new K row (into the cache and, for the fragments already loaded, knew) and V row. The V
+// values are loaded first: behind the K stores, which might alias, each would wait for them.
 __device__ __forceinline__ void make_kv_row(const AttnArgs& a, const uint16_t* prow, int pos, int lrow, int j, int slot,
                                             uint16_t* knew) {
     const int lane = threadIdx.x & 63;
+    uint16_t v[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) v[w] = prow[kAttnVOff + j * 256 + lane + 64 * w];
     float o[4];
     head_norm_rope_wave(a, prow + kAttnKOff + j * 256, a.k_norm, pos, o);
     const size_t base = lrow * a.kv_lane + a.kv_layer_off + (size_t)j * a.cap * 256;
@@ -261,7 +269,7 @@ __device__ __forceinline__ void make_kv_row(const AttnArgs& a, const uint16_t* p
         const uint16_t kb = f2bf(o[w]);
         knew[d] = kb;
         a.kc[base + kv_tiled_offset(slot, d)] = kb;
-        a.vc[base + kv_v8_offset(slot, d)] = prow[kAttnVOff + j * 256 + d];
+        a.vc[base + kv_v8_offset(slot, d)] = v[w];
     }
 }
 // The new K row in place of the fragments of sub-tile st in the lanes that hold its row (selects: with
@@ -477,6 +485,12 @@ __device__ __forceinline__ void store_gated(const AttnArgs& a, int r, int j, int
             po[h * 256 + 16 * i] = f2bf(rbf(acc[i][h]) * rbf(sigmoid_f(bf2f(graw[i][h]))));
 }
 
+// A part's partial sums: [row][part][kv head][dim][4 heads], so a lane's four heads of one dim
+// (one MFMA accumulator) are one 16-byte store.
+__device__ __forceinline__ size_t part_offset(const AttnArgs& a, int r, int pc, int j, int d) {
+    return ((((size_t)r * a.max_chunks * 2 + pc) * kNkv + j) * 256 + d) * 4;
+}
+
 // Split path, one block per (row, kv head, part): wave w takes dims 64w .. +64.
 __global__ void __launch_bounds__(256) attn_pv(AttnArgs a) {
     __shared__ uint16_t pl[16 * kPlStride];
@@ -495,20 +509,26 @@ __global__ void __launch_bounds__(256) attn_pv(AttnArgs a) {
     q35_f32x4 out[4];
     pv_mfma(pl, 4, vf, out);
     if (lane < 16) {
-        float* pp = a.part + (((size_t)r * a.max_chunks * 2 + pc) * kNq + 4 * j) * 256 + 64 * wv + lane;
+        float* pp = a.part + part_offset(a, r, pc, j, 64 * wv + lane);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int h = 0; h < 4; ++h) pp[h * 256 + 16 * i] = out[i][h];
+        for (int i = 0; i < 4; ++i) *(q35_f32x4*)(pp + 64 * i) = out[i];
     }
 }
 
-// Sum of the 128-slot partials in part order, bf16, times bf16(sigmoid(gate)).
-__global__ void __launch_bounds__(256) attn_combine(AttnArgs a) {
-    const int r = blockIdx.x, qh = blockIdx.y, tid = threadIdx.x;
+// Sum of the 128-slot partials in part order, bf16, times bf16(sigmoid(gate)). Block (row, kv
+// head, 64 dims), a thread per (dim, head). whole: the most parts of a lane whose pairs
+// attn_seg_pv finishes by itself (its T rows' last slot decides; 0: none).
+__global__ void __launch_bounds__(256) attn_combine(AttnArgs a, int whole) {
+    const int r = blockIdx.x, j = blockIdx.y >> 2, tid = threadIdx.x, h = tid & 3;
+    const int d = (blockIdx.y & 3) * 64 + (tid >> 2);
     const int nparts = a.rm.slot[r] / kPart + 1;
-    const float* pp = a.part + ((size_t)r * a.max_chunks * 2 * kNq + qh) * 256 + tid;
-    const uint16_t graw = a.proj[(size_t)r * kAttnInRows + qh * 512 + 256 + tid];
+    if (whole) {
+        int last = 0;
+        for (int t = 0, r0 = r / a.T * a.T; t < a.T; ++t) last = max(last, a.rm.slot[r0 + t]);
+        if (last / kPart + 1 <= whole) return;
+    }
+    const float* pp = a.part + part_offset(a, r, 0, j, d) + h;
+    const uint16_t graw = a.proj[(size_t)r * kAttnInRows + (4 * j + h) * 512 + 256 + d];
     float acc = 0.f;
     // 40 parts per round (a 5,120-slot context in one), all loads issued before the adds:
     // unconditional from clamped part indices, so no branch makes the compiler wait per load
@@ -522,7 +542,7 @@ __global__ void __launch_bounds__(256) attn_combine(AttnArgs a) {
     }
     const float o = rbf(acc);
     const float g = rbf(sigmoid_f(bf2f(graw)));
-    a.out[(size_t)r * 2048 + qh * 256 + tid] = f2bf(o * g);
+    a.out[(size_t)r * 2048 + (4 * j + h) * 256 + d] = f2bf(o * g);
 }
 
 // ---------------------------------------------------------------- split path, 4-wave blocks
@@ -651,11 +671,9 @@ __global__ void __launch_bounds__(64) attn_pv4(AttnArgs a) {
     q35_f32x4 out[4];
     pv_mfma(pl, 4, vf, out);
     if (tid < 16) {
-        float* pp = a.part + (((size_t)r * a.max_chunks * 2 + pc) * kNq + 4 * j) * 256 + dq * 64 + tid;
+        float* pp = a.part + part_offset(a, r, pc, j, dq * 64 + tid);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int h = 0; h < 4; ++h) pp[h * 256 + 16 * i] = out[i][h];
+        for (int i = 0; i < 4; ++i) *(q35_f32x4*)(pp + 64 * i) = out[i];
     }
 }
 
@@ -1039,6 +1057,261 @@ __global__ void __launch_bounds__(64 * W) attn_rows(AttnArgs a) {
     if (tg < T) store_gated<NTL>(a, r0 + tg, j, 16 * NTL * wv + (lane & 15), acc);
 }
 
+// ---------------------------------------------------------------- verify rows by segments
+// T = 2 or 3 rows of a lane at few lanes: the lane's K/V stream once for all of its rows, as in
+// attn_rows, but cut into segments of a (lane, kv head) pair, so that a few long contexts fill the
+// CUs (the split path's blocks take one row each and read the K/V T times):
+//   attn_seg_scores  (pair, 256-slot chunk): wave w scores slice w of the chunk for every row; q
+//                    and, with PREP, the chunk's new K / V rows are made by the block; scores and
+//                    slice stats leave as whole lines
+//   attn_seg_pv      (pair, kSegParts parts): attn_rows' P.V over the segment's parts; a pair of one
+//                    segment is finished here, longer ones leave their parts to attn_combine
+// Slices, parts and their sums are the other forms', so the results are the same bits. Bound by
+// the K/V stream plus the scores' and parts' round trip (a tenth of its bytes, but a fifth of the
+// time: writes between the reads cost HBM several times their size). us, split path -> segments:
+// 24 lanes x 3 rows x 8,192 slots 277 -> 127, ragged 178 -> 100; 16 x 3 x 2,000 65 -> 50.
+constexpr int kSegRow = 68;                              // floats of a slice's (row, head) in LDS: 64 scores, max, sum
+constexpr int kSegParts = 4;                             // parts (128 slots) of a P.V segment
+
+// Block -> (pair, segment): a pair's segments in consecutive blocks of one XCD, so that lanes of
+// different lengths load the XCDs alike.
+__device__ __forceinline__ bool seg_of(const AttnArgs& a, int nseg, int& pr, int& seg) {
+    const int k = blockIdx.x >> 3;
+    pr = (k / nseg) * 8 + (blockIdx.x & 7);
+    seg = k % nseg;
+    return pr < a.R / a.T * kNkv;
+}
+
+template <int T, bool PREP>
+__global__ void __launch_bounds__(256, 2) attn_seg_scores(AttnArgs a, int nseg) {
+    constexpr int NU = (T + 1) / 2;                     // q tiles
+    __shared__ uint16_t qbuf[NU][16][256];
+    __shared__ uint16_t knew[T][256];
+    __shared__ float ss_all[4][T][4][kSegRow];          // each wave's slice, then whole lines to memory
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, n = lane & 15, g = lane >> 4;
+    int pr, c;
+    if (!seg_of(a, nseg, pr, c)) return;
+    const int j = pr % kNkv, r0 = (pr / kNkv) * T;
+    int slot_t[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) slot_t[t] = a.rm.slot[r0 + t];
+    int slot = slot_t[0];
+#pragma unroll
+    for (int t = 1; t < T; ++t) slot = max(slot, slot_t[t]);
+    if (c * kChunk > slot) return;
+    const int lrow = a.rm.lane[r0], q = 4 * c + wv, t0 = q * 64;
+    q35_u32x4 kf[2][8];
+    load_k_sub<true>(a, lrow, j, q, 0, slot, kf[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_k_sub<true>(a, lrow, j, q, 1, slot, kf[1]);
+    // q fragments: tile u, column 8 (t % 2) + h = bf16(q) of row t = 2u + t % 2, head h, and + 4 its
+    // low part (a missing row's columns stay as they are); wave w makes head w of every row
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const int col = 8 * (t & 1) + wv;
+        float o[4];
+        if constexpr (PREP) {
+            head_norm_rope_wave(a, a.proj + (size_t)(r0 + t) * kAttnInRows + (4 * j + wv) * 512, a.q_norm,
+                                a.rm.pos[r0 + t], o);
+        } else {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) o[w] = a.q[((size_t)(r0 + t) * kNq + 4 * j + wv) * 256 + lane + 64 * w];
+        }
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const uint16_t hi = f2bf(o[w]);
+            qbuf[t >> 1][col][lane + 64 * w] = hi;
+            qbuf[t >> 1][col + 4][lane + 64 * w] = f2bf(o[w] - bf2f(hi));
+        }
+    }
+    if (PREP && wv < T) {                               // row wv's new K / V row, if it is in this chunk
+        const int sl = a.rm.slot[r0 + wv];
+        if (sl / kChunk == c)
+            make_kv_row(a, a.proj + (size_t)(r0 + wv) * kAttnInRows, a.rm.pos[r0 + wv], lrow, j, sl, knew[wv]);
+    }
+    __syncthreads();
+    if (t0 > slot) return;
+    q35_u32x4 qf[NU][8];
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int s = 0; s < 8; ++s) qf[u][s] = *(const q35_u32x4*)&qbuf[u][n][s * 32 + g * 8];
+    const int tr = n >> 3;                               // this lane's row within a tile: 2u + tr
+    int lslot[NU];                                       // that row's slot (-1: no such row)
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+        const int ta = 2 * u, tb = 2 * u + 1 < T ? 2 * u + 1 : 2 * u;
+        lslot[u] = tr == 0 ? slot_t[ta] : 2 * u + 1 < T ? slot_t[tb] : -1;
+    }
+    float(*ss)[4][kSegRow] = ss_all[wv];
+    float sv[NU][4][4];
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+        if (PREP) {                                      // new K rows: their loads may be stale
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+                if (slot_t[t] >> 4 == 4 * q + st && n == (slot_t[t] & 15)) {
+#pragma unroll
+                    for (int s = 0; s < 8; ++s) kf[st & 1][s] = *(const q35_u32x4*)&knew[t][s * 32 + g * 8];
+                }
+        }
+        q35_f32x4 acc[NU];
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            acc[u] = (q35_f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(q35_bf16x8*)&kf[st & 1][s], *(const q35_bf16x8*)&qf[u][s], acc[u], 0, 0, 0);
+        }
+        if (st < 2) load_k_sub<true>(a, lrow, j, q, st + 2, slot, kf[st & 1]);
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            q35_f32x4 scv;
+            const int t = 2 * u + tr, tt0 = t0 + st * 16 + 4 * g;
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+                const float lo = row_down4(acc[u][rr]);   // lanes with n % 8 < 4 add the q_lo column
+                const float sc = (acc[u][rr] + lo) * 0.0625f;
+                const bool ok = (n & 7) < 4 && tt0 + rr <= lslot[u];
+                sv[u][st][rr] = ok ? sc : -INFINITY;
+                scv[rr] = sc;
+            }
+            if ((n & 7) < 4 && t < T) *(q35_f32x4*)&ss[t][n & 3][st * 16 + 4 * g] = scv;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+        float m = -INFINITY;
+#pragma unroll
+        for (int st = 0; st < 4; ++st)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) m = fmaxf(m, sv[u][st][rr]);
+        m = fmaxf(m, xor16(m));
+        m = fmaxf(m, xor32(m));
+        float e = 0.f;
+#pragma unroll
+        for (int st = 0; st < 4; ++st)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) e += sv[u][st][rr] > -INFINITY ? expf(sv[u][st][rr] - m) : 0.f;
+        e += xor16(e);
+        e += xor32(e);
+        if (g == 0 && (n & 7) < 4 && 2 * u + tr < T) *(float2*)&ss[2 * u + tr][n & 3][64] = make_float2(m, e);
+    }
+    // a row's slice of scores as one contiguous KiB (slots past the row's last are never read), in
+    // this form's own order of the scratch: [row][kv head][slice][head][64 slots]
+    wave_sync();
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        if (t0 > slot_t[t]) continue;
+        *(q35_f32x4*)(a.sc + (((size_t)(r0 + t) * kNkv + j) * (a.sc_ld / 64) + q) * 256 + lane * 4) =
+            *(const q35_f32x4*)&ss[t][lane >> 4][(lane & 15) * 4];
+        if (lane < 4)
+            *(float2*)(a.stats + ((size_t)(r0 + t) * kNq + 4 * j + lane) * a.max_chunks * 8 + 2 * q) = *(const float2*)&ss[t][lane][64];
+    }
+}
+
+// kSegParts x T x 4 KiB of dynamic LDS when a pair can have more than one segment
+template <int T>
+__global__ void __launch_bounds__(256, 2) attn_seg_pv(AttnArgs a, int nseg) {
+    __shared__ uint16_t pl[16 * kPlStride];
+    __shared__ float ml_all[T][4][2];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, g = lane >> 4;
+    int pr, p0;
+    if (!seg_of(a, nseg, pr, p0)) return;
+    p0 *= kSegParts;
+    const int j = pr % kNkv, r0 = (pr / kNkv) * T;
+    int slot_t[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) slot_t[t] = a.rm.slot[r0 + t];
+    int slot = slot_t[0];
+#pragma unroll
+    for (int t = 1; t < T; ++t) slot = max(slot, slot_t[t]);
+    const int np = slot / kPart + 1, p1 = min(p0 + kSegParts, np);
+    if (p0 >= np) return;
+    const int lrow = a.rm.lane[r0];
+    const size_t sst = (size_t)a.max_chunks * 8;
+    // the thread's two scores of a part per row (head idx / 128, slot idx % 128), loaded two parts
+    // ahead and issued before that part's V (see attn_rows)
+    auto load_scores = [&](int pc, float (&sr)[T][2]) {
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int idx = tid + q * 256, i = idx >> 7, tt = idx & 127;
+                const int ts = min(pc * kPart + tt, slot);
+                sr[t][q] = a.sc[(((size_t)(r0 + t) * kNkv + j) * (a.sc_ld / 64) + (ts >> 6)) * 256 + i * 64 + (ts & 63)];
+            }
+    };
+    q35_u32x4 vfa[4][4], vfb[4][4];
+    float sra[T][2], srb[T][2];
+    load_scores(p0, sra);
+    __builtin_amdgcn_sched_barrier(0);
+    load_vf(a, lrow, j, p0, slot, 4 * wv, vfa);
+    __builtin_amdgcn_sched_barrier(0);
+    load_scores(p0 + 1, srb);
+    __builtin_amdgcn_sched_barrier(0);
+    load_vf(a, lrow, j, p0 + 1, slot, 4 * wv, vfb);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+        softmax_ml(a.stats + ((size_t)(r0 + t) * kNq + 4 * j) * sst, sst, slot_t[t] / 64 + 1, ml_all[t]);
+    const int myslot = g == 0 ? slot_t[0] : g == 1 ? slot_t[T > 1 ? 1 : 0] : slot_t[T > 2 ? 2 : 0];
+    const bool whole = np <= kSegParts;                          // block-uniform: no other segment of this pair
+    // the parts' sums wait in LDS, [P][T][4 waves][4 tiles][16 dims][4 heads], for the segment's end
+    // (see attn_seg_scores)
+    extern __shared__ __attribute__((aligned(16))) float seg_lds[];
+    float* mypart = seg_lds + (min(g, T - 1) * 4 + wv) * 256 + (lane & 15) * 4;
+    q35_f32x4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = (q35_f32x4){0.f, 0.f, 0.f, 0.f};
+    auto part = [&](int pc, q35_u32x4 (&vf)[4][4], float (&sr)[T][2], auto more) {
+        lds_barrier();          // ml is in; every wave is done with the previous part's weights
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const int nn = min(kPart, slot_t[t] + 1 - pc * kPart);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int idx = tid + q * 256, i = idx >> 7, tt = idx & 127;
+                pl[(4 * t + i) * kPlStride + tt] = tt < nn ? f2bf(expf(sr[t][q] - ml_all[t][i][0]) / ml_all[t][i][1]) : (uint16_t)0;
+            }
+        }
+        lds_barrier();
+        if (pc == np - 1) mask_vf(pc, slot, vf);
+        q35_f32x4 out[4];
+        pv_mfma(pl, 4 * T, vf, out);
+        if (decltype(more)::value) {
+            load_scores(pc + 2, sr);
+            load_vf(a, lrow, j, pc + 2, slot, 4 * wv, vf);
+        }
+        // lane (n, g) holds row g's four heads of dim 16 (4 wv + i) + n
+        const bool mine = g < T && pc < myslot / kPart + 1;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (!whole && g < T) *(q35_f32x4*)(mypart + (pc - p0) * T * 1024 + i * 64) = out[i];
+            if (mine) acc[i] += out[i];
+        }
+    };
+    int pc = p0;
+    for (; pc + 2 < p1; pc += 2) {
+        part(pc, vfa, sra, std::true_type{});
+        part(pc + 1, vfb, srb, std::true_type{});
+    }
+    part(pc, vfa, sra, std::false_type{});
+    if (pc + 1 < p1) part(pc + 1, vfb, srb, std::false_type{});
+    if (!whole) {
+        wave_sync();
+        for (pc = p0; pc < p1; ++pc)
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+                if (pc < slot_t[t] / kPart + 1)
+                    *(q35_f32x4*)(a.part + part_offset(a, r0 + t, pc, j, 64 * wv) + lane * 4) =
+                        *(const q35_f32x4*)(seg_lds + ((pc - p0) * T + t) * 1024 + wv * 256 + lane * 4);
+        return;
+    }
+    if (g < T) store_gated<4>(a, r0 + g, j, 64 * wv + (lane & 15), acc);
+}
+
 // ---------------------------------------------------------------- prompt waves (flash form)
 // A prompt wave of one lane (T >= 64 rows at consecutive slots): all of its rows read the
 // same K/V, so a block takes 16 rows x the 4 q heads of one kv head (64 query columns) and
@@ -1344,6 +1617,18 @@ static bool use_rows(const AttnArgs& a) {
     if (a.force != kAttnAuto) return false;
     return a.rows_form && shape && a.R >= 192;
 }
+// Verify rows below the rows form's line: by segments where the lanes' capacities together make
+// enough work for two more launches and the fused form, a block per row, is no better. us, fused ->
+// segments: 31 lanes x 3 rows x 4,000 slots 98 -> 91, ragged 81 -> 70; 31 x 2 x 4,000 99 -> 87; 64 x 2 x
+// 4,000 125 -> 145, 32 x 3 x 3,000 79 -> 87, 31 x 3 x 1,000 42 -> 43. Split path -> segments: 24 x 3 x
+// 8,192 277 -> 127, 16 x 3 x 2,000 65 -> 50, 8 x 3 x 4,000 61 -> 48, 8 x 3 x 2,000 44 -> 45; two rows (the
+// split path reads the K/V only twice then): 24 x 2 x
+// 8,192 186 -> 119, 3 x 2 x 32,768 124 -> 93, 16 x 2 x 2,000 50 -> 56, 8 x 2 x 4,000 49 -> 56.
+static bool use_seg(const AttnArgs& a) {
+    if (a.force != kAttnAuto || (a.T != 2 && a.T != 3) || a.R % a.T || use_rows(a)) return false;
+    if (use_fused(a) && (a.R >= 96 || a.cap < 2048)) return false;
+    return (long long)(a.R / a.T) * a.cap >= (a.T == 2 ? 90000 : 30000);
+}
 static bool use_prompt(const AttnArgs& a) {
     const bool shape = a.T >= 64 && a.R == a.T;
     if (a.force == kAttnPrompt) return shape;
@@ -1352,7 +1637,7 @@ static bool use_prompt(const AttnArgs& a) {
 }
 
 // The form makes q and the new K / V rows itself: the split path with one row per lane; the fused
-// form with one row per lane and the rows form, whose blocks read only rows they make, as long as
+// form with one row per lane, the rows form and the segments, whose blocks read only rows they make, as long as
 // no lane occurs twice (another row's block would append to the same lane). The fused form up to
 // 600,000 slots in all: there the launch it saves is 2 .. 8 % (us, attn_prep -> folded: 256 lanes x
 // 1,000 slots 117.4 -> 113.9, 130 x 4,000 223 -> 212); beyond it a full chip streaming at the HBM
@@ -1360,7 +1645,7 @@ static bool use_prompt(const AttnArgs& a) {
 // -> 350). The rows form gains everywhere (250 lanes x 3 rows x 2,000: 200 -> 198, ragged 158 -> 151).
 static bool prep_folded(const AttnArgs& a) {
     if (use_prompt(a)) return false;
-    if (use_rows(a)) return a.distinct;
+    if (use_rows(a) || use_seg(a)) return a.distinct;
     return a.T == 1 && (!use_fused(a) || (a.distinct && (long long)a.R * a.cap <= 600000));
 }
 // the split path's part of that
@@ -1406,6 +1691,19 @@ hipError_t launch_attn_core(const AttnArgs& a, hipStream_t st) {
     }
         Q35_ROWS(2, 8) Q35_ROWS(3, 8) Q35_ROWS(2, 4) Q35_ROWS(3, 4)
 #undef Q35_ROWS
+    } else if (use_seg(a)) {
+        const int pairs = (a.R / a.T * kNkv + 7) / 8 * 8, ns = a.max_chunks;
+        const int np = ((a.cap + kPart - 1) / kPart + kSegParts - 1) / kSegParts;
+        const size_t lp = np > 1 ? (size_t)kSegParts * a.T * 4096 : 0;
+#define Q35_SEG(TV)                                                                                              \
+    if (a.T == TV) {                                                                                             \
+        if (prep_folded(a)) hipLaunchKernelGGL((attn_seg_scores<TV, true>), dim3(pairs * ns), dim3(256), 0, st, a, ns); \
+        else hipLaunchKernelGGL((attn_seg_scores<TV, false>), dim3(pairs * ns), dim3(256), 0, st, a, ns);        \
+        hipLaunchKernelGGL((attn_seg_pv<TV>), dim3(pairs * np), dim3(256), lp, st, a, np);                       \
+    }
+        Q35_SEG(2) Q35_SEG(3)
+#undef Q35_SEG
+        if (np > 1) hipLaunchKernelGGL(attn_combine, dim3(a.R, kNq), dim3(256), 0, st, a, kSegParts);
     } else if (use_fused(a)) {
         if (a.T < 1 || a.R % a.T) return hipErrorInvalidValue;
         const int pairs = a.R / a.T * kNkv;
@@ -1436,7 +1734,7 @@ hipError_t launch_attn_core(const AttnArgs& a, hipStream_t st) {
                 hipLaunchKernelGGL(attn_scores, dim3(a.R, kNkv, a.max_chunks * 4), dim3(64), 0, st, a);
             hipLaunchKernelGGL(attn_pv, dim3(a.R, kNkv, a.max_chunks * 2), dim3(256), 0, st, a);
         }
-        hipLaunchKernelGGL(attn_combine, dim3(a.R, kNq), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(attn_combine, dim3(a.R, kNq), dim3(256), 0, st, a, 0);
     }
     return hipGetLastError();
 }

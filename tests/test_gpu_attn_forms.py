@@ -46,6 +46,34 @@ def test_folded_prep_equals_split(harness, B, T):
         assert np.array_equal(k2, k) and np.array_equal(v2, v), (lanes[i], pos[i])
 
 
+@pytest.mark.parametrize("T", [2, 3])
+def test_segments_equal_split(T):
+    """Verify rows of 31 lanes x 3,000 slots (the segment form) at the borders of its chunks (256
+    slots) and P.V segments (512), rows that straddle them, a lane of one segment and an empty one,
+    and with a lane named twice (q and K / V rows from the prep launch)."""
+    h = Harness(3000, 128)
+    try:
+        pos = [0, 1, 62, 126, 253, 254, 255, 256, 509, 510, 511, 512, 513, 1022, 1023, 1024, 1535, 2047, 2048, 2303,
+               2558, 2815, 2990, 3000 - T]
+        pos += [int(p) for p in np.random.default_rng(T).integers(0, 2990, 7)]
+        lanes = np.random.default_rng(T).permutation(256)[:31].tolist()
+        want = h.run(lanes, pos, T, 1)
+        for i in range(31):
+            for n in "kv":
+                full = np.asarray(h.s.read(lanes[i], n, pos[i] + T))
+                full[LAYER][:, pos[i]:pos[i] + T] = 0
+                h.s.write(lanes[i], n, full, pos[i] + T)
+        assert np.array_equal(h.run(lanes, pos, T, 0), want)
+        for i in (0, 6, 11, 23):
+            h.check_lane(i, lanes[i], pos[i], T, want)
+        lanes[5] = lanes[6]                 # a second group of the lane, right after the first
+        pos[5] = pos[6] + T
+        assert np.array_equal(h.run(lanes, pos, T, 0), h.run(lanes, pos, T, 1))
+    finally:
+        h.s.close()
+        h.e.close()
+
+
 @pytest.mark.parametrize("B, T", [(64, 1), (130, 1), (128, 3)])
 def test_lane_named_twice(harness, B, T):
     """Two row groups of one lane, the second right after the first: every row reads both."""
