@@ -5,7 +5,7 @@ slice, a 128-slot part, a 256-slot chunk), and with a lane named twice (no foldi
 import numpy as np
 import pytest
 
-from test_gpu_attn_op import Harness, LAYER
+from test_gpu_attn_op import Harness, LAYER, bf16_val
 
 pytestmark = pytest.mark.gpu
 EDGES = [0, 1, 14, 15, 16, 17, 62, 63, 64, 65, 126, 127, 128, 254, 255, 256, 257, 510, 511, 512, 513, 1020, 1021]
@@ -69,6 +69,37 @@ def test_segments_equal_split(T):
         lanes[5] = lanes[6]                 # a second group of the lane, right after the first
         pos[5] = pos[6] + T
         assert np.array_equal(h.run(lanes, pos, T, 0), h.run(lanes, pos, T, 1))
+    finally:
+        h.s.close()
+        h.e.close()
+
+
+@pytest.mark.parametrize("T", [2, 3])
+@pytest.mark.parametrize("form, rows", [(5, 1), (5, 2), (0, 2)])
+def test_later_rows_stay_out_of_earlier_ones(T, form, rows):
+    """A non-finite row (its V infinite, or all of its projection NaN) is cached behind the lane's
+    earlier rows only: those keep the split form's bits, which attends over slots 0 .. p + t. Rows that
+    lie in one part (128 slots), end one and straddle two; the rows form in both block sizes and,
+    through auto, the segments (whose P.V segments are 512 slots: a lane of one, lanes of several)."""
+    h = Harness(8192, 192)
+    try:
+        h.e.set_option("attn_rows", rows)
+        pos = [0, 1, 5, 63, 124, 125, 126, 127, 128, 254, 255, 256, 509, 510, 511, 512, 1021, 1022, 1023, 1024]
+        pos += [8000 - 131 * i for i in range(20)]                     # enough slots in all for the segments
+        n = len(pos)
+        lanes = np.random.default_rng(T).permutation(256)[:n].tolist()
+        bits = h.proj.view(h.torch.int16)
+        good = bits.clone()
+        for bad in range(1, T):
+            for cols, value in ((slice(4608, 5120), 0x7F80), (slice(0, 5120), 0x7FC0)):
+                bits.copy_(good)
+                bits[bad:n * T:T, cols] = value
+                want = h.run(lanes, pos, T, 1).reshape(n, T, 2048)
+                got = h.run(lanes, pos, T, form).reshape(n, T, 2048)
+                assert np.isfinite(bf16_val(want[:, :bad])).all()
+                assert np.array_equal(got[:, :bad], want[:, :bad]), (bad, hex(value), np.argwhere(
+                    (got[:, :bad] != want[:, :bad]).any(-1))[:8].tolist())
+                assert np.array_equal(np.isfinite(bf16_val(got)), np.isfinite(bf16_val(want)))
     finally:
         h.s.close()
         h.e.close()
