@@ -1681,20 +1681,18 @@ static bool use_prompt(const AttnArgs& a) {
     return a.prompt_flash && shape;
 }
 
-// The form makes q and the new K / V rows itself: the split path with one row per lane; the fused
-// form with one row per lane, the rows form and the segments, whose blocks read only rows they make, as long as
-// no lane occurs twice (another row's block would append to the same lane). The fused form up to
+// The form makes q and the new K / V rows itself: the split and the fused form with one row per lane, the
+// rows form and the segments, whose blocks read only rows they make, as long as no lane occurs twice
+// (another row's block would append to the lane while this one reads it). The fused form up to
 // 600,000 slots in all: there the launch it saves is 2 .. 8 % (us, attn_prep -> folded: 256 lanes x
 // 1,000 slots 117.4 -> 113.9, 130 x 4,000 223 -> 212); beyond it a full chip streaming at the HBM
 // rate pays more for every block's appended rows at once (224 x 3,000 237 -> 242, 240 x 4,000 323
 // -> 350). The rows form gains everywhere (250 lanes x 3 rows x 2,000: 200 -> 198, ragged 158 -> 151).
 static bool prep_folded(const AttnArgs& a) {
-    if (use_prompt(a)) return false;
-    if (use_rows(a) || use_seg(a)) return a.distinct;
-    return a.T == 1 && (!use_fused(a) || (a.distinct && (long long)a.R * a.cap <= 600000));
+    if (use_prompt(a) || !a.distinct) return false;
+    if (use_rows(a) || use_seg(a)) return true;
+    return a.T == 1 && (!use_fused(a) || (long long)a.R * a.cap <= 600000);
 }
-// the split path's part of that
-static bool prep_in_scores(const AttnArgs& a) { return a.T == 1; }
 
 bool attn_prompt_form(const AttnArgs& a) { return use_prompt(a); }
 
@@ -1767,13 +1765,13 @@ hipError_t launch_attn_core(const AttnArgs& a, hipStream_t st) {
         }
     } else {
         if (a.force == kAttnSplit4 || (a.force != kAttnSplit && a.split4)) {
-            if (prep_in_scores(a))
+            if (prep_folded(a))
                 hipLaunchKernelGGL(attn_scores4<true>, dim3(a.R, kNkv, a.max_chunks * 4), dim3(256), 0, st, a);
             else
                 hipLaunchKernelGGL(attn_scores4<false>, dim3(a.R, kNkv, a.max_chunks * 4), dim3(256), 0, st, a);
             hipLaunchKernelGGL(attn_pv4, dim3(a.R, kNkv, a.max_chunks * 8), dim3(64), 0, st, a);
         } else {
-            if (prep_in_scores(a))
+            if (prep_folded(a))
                 hipLaunchKernelGGL(attn_scores_prep, dim3(a.R, kNkv, a.max_chunks * 4), dim3(64), 0, st, a);
             else
                 hipLaunchKernelGGL(attn_scores, dim3(a.R, kNkv, a.max_chunks * 4), dim3(64), 0, st, a);

@@ -23,6 +23,29 @@ def rows_at(h, lane, p, T):
     return [np.asarray(h.s.read(lane, n, p + T))[LAYER][:, p:p + T].copy() for n in "kv"]
 
 
+def clear_slots(h, lane, p, n):
+    """Zero K and V in slots p .. p + n: the rows a call appends there must be its own."""
+    for kv in "kv":
+        full = np.asarray(h.s.read(lane, kv, p + n))
+        full[LAYER][:, p:p + n] = 0
+        h.s.write(lane, kv, full, p + n)
+
+
+def run_from(h, row, lanes, pos, T, form):
+    """Harness.run on the projection rows from `row` on."""
+    h.out.fill_(0)
+    h.e.op_attn_decode(h.s, LAYER, lanes, pos, T, h.proj[row:].data_ptr(), h.qn.data_ptr(), h.kn.data_ptr(),
+                       h.out.data_ptr(), form)
+    return h.out[:len(lanes) * T].view(h.torch.int16).cpu().numpy().view(np.uint16).copy()
+
+
+def prepared_q(h):
+    """Row 0's q at position 500 in the q scratch (four rows of a lane always take the prep launch): a
+    later call's prep launch writes its own over it, a form that makes q in its blocks leaves it."""
+    h.run([1], [500], 4, 1)
+    return h.e.read_scratch("q", (2048,), np.float32)
+
+
 @pytest.mark.parametrize("T", [1, 2, 3])
 @pytest.mark.parametrize("B", [2, 63, 64, 96, 128, 129, 256])
 def test_folded_prep_equals_split(harness, B, T):
@@ -105,10 +128,19 @@ def test_later_rows_stay_out_of_earlier_ones(T, form, rows):
         h.e.close()
 
 
-@pytest.mark.parametrize("B, T", [(64, 1), (130, 1), (128, 3)])
-def test_lane_named_twice(harness, B, T):
-    """Two row groups of one lane, the second right after the first: every row reads both."""
+@pytest.mark.parametrize("B, T, form", [(2, 1, 0), (2, 1, 1), (2, 1, 2), (63, 1, 0), (64, 1, 0), (64, 1, 3), (130, 1, 0),
+                                         (130, 1, 4), (2, 3, 0), (2, 2, 5), (96, 2, 5), (128, 3, 0)])
+def test_lane_named_twice(harness, B, T, form):
+    """Two row groups of one lane, the second right after the first and reading its rows: every row
+    equals the two groups' calls one after the other (slots to be appended cleared before each), and
+    q comes from the prep launch, which appends every K / V row before any block reads one."""
     h = harness
     lanes = list(range(B - 1)) + [0]
     pos = [40] * (B - 1) + [40 + T]
-    assert np.array_equal(h.run(lanes, pos, T, 0)[:T * (B - 1)], h.run(lanes, pos, T, 3)[:T * (B - 1)])
+    clear_slots(h, 0, 40, 2 * T)
+    want = [run_from(h, 0, lanes[:-1], pos[:-1], T, 1), run_from(h, (B - 1) * T, lanes[-1:], pos[-1:], T, 1)]
+    clear_slots(h, 0, 40, 2 * T)
+    before = prepared_q(h)
+    got = h.run(lanes, pos, T, form)
+    assert np.array_equal(got, np.concatenate(want))
+    assert not np.array_equal(h.e.read_scratch("q", (2048,), np.float32), before)
