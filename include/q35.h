@@ -254,10 +254,11 @@ int q35_kprof_read(q35_engine* e, float* total_ms, int* launches);
  * the block, one chain for the add+norm; default 1,024), "attn_split4" (split attention path
  * in 4-wave score blocks and dim-quarter P.V blocks), "attn_pair" (default 1: the fused
  * attention of one row per lane above 128 lanes runs two (row, kv head) items per block when
- * their LDS fits the CU, so the two items on a CU finish together), "attn_rows" (default 1: MTP
+ * their LDS fits the CU, so the two items on a CU finish together), "attn_rows" (default 2: MTP
  * verify bodies of 2-3 rows per lane from 192 rows on run one attention block per (lane, kv
- * head) for all of the lane's rows, streaming its K/V once), "gdn_rows" (default 1: those verify
- * bodies' GDN layers in the persistent kernel, the next (lane, head) item prefetched),
+ * head) for all of the lane's rows, streaming its K/V once, unless a few long lanes hold most
+ * of the cached slots; 1: the same in 4-wave blocks, two per CU; 0: off), "gdn_rows" (default
+ * 1: the GDN layers of verify bodies in the persistent kernel, the next (lane, head) item prefetched),
  * "gdn_defer" (0 .. 4, default 3: a decode
  * step keeps each lane's GDN state update as pending factors for up to this many steps and
  * writes the state with the next one; 0 writes it every step). Not bit-identical, a different

@@ -1101,9 +1101,9 @@ __global__ void __launch_bounds__(64 * W) attn_rows(AttnArgs a) {
 }
 
 // ---------------------------------------------------------------- verify rows by segments
-// T = 2 or 3 rows of a lane at few lanes: the lane's K/V stream once for all of its rows, as in
-// attn_rows, but cut into segments of a (lane, kv head) pair, so that a few long contexts fill the
-// CUs (the split path's blocks take one row each and read the K/V T times):
+// T = 2 or 3 rows of a lane at few lanes, or at many of which a few are long: the lane's K/V stream once
+// for all of its rows, as in attn_rows, but cut into segments of a (lane, kv head) pair, so that a few
+// long contexts fill the CUs (the split path's blocks take one row each and read the K/V T times):
 //   attn_seg_scores  (pair, 256-slot chunk): wave w scores slice w of the chunk for every row; q
 //                    and, with PREP, the chunk's new K / V rows are made by the block; scores and
 //                    slice stats leave as whole lines
@@ -1652,27 +1652,37 @@ static bool use_fused2(const AttnArgs& a) {
 // A lane's 2-3 verify rows in one block from 192 rows on: the K/V stream once instead of once per
 // row. us, one block per row -> rows form: 100 lanes x 2 x 3,000 171 -> 123, ragged 143 -> 101; 64 x 3
 // x 4,000 185 -> 145, ragged 138 -> 125; 64 x 3 x 1,000 58.6 -> 59.3, 64 x 2 x 4,000 125 -> 127, 32 x 3 x
-// 4,000 99 -> 124.
+// 4,000 99 -> 124. A block streams its lane's slots at 22.5 ns each, the full chip all lanes' at 0.45, so
+// with less than 40 of the longest lane's slots in all the longest lane alone sets the time, and the
+// segments cut it up. us, rows form -> segments: 64 x 3, 1 lane of 4,096 and the others of 128 120 -> 62,
+// of 32,768 and 1,000 741 -> 139; a third of 80 lanes of 4,000, the others of 500 (33 times) 126 -> 112; 64
+// lanes of 512 .. 4,096 (36) 126 -> 118, 80 (45) 131 -> 134; below 3,000 slots the two more launches
+// weigh more: 64 of 250 .. 2,000 78 -> 82.
 static int rows_w(const AttnArgs& a) { return a.rows_form == 2 ? 8 : 4; }
+static bool uneven(const AttnArgs& a) { return a.ctx_max >= 3000 && a.ctx_sum < 40ll * a.ctx_max; }
 static bool use_rows(const AttnArgs& a) {
     // the slice stats (and the tail) fit the block's dynamic LDS
     const bool shape = (a.T == 2 || a.T == 3) && a.R % a.T == 0 &&
                        rows_lds_bytes(a.T, a.max_chunks, rows_w(a)) <= (rows_w(a) == 8 ? (size_t)kRowsLdsDyn8 : 65536);
     if (a.force == kAttnRows) return shape;
     if (a.force != kAttnAuto) return false;
-    return a.rows_form && shape && a.R >= 192;
+    return a.rows_form && shape && a.R >= 192 && !uneven(a);
 }
-// Verify rows below the rows form's line: by segments where the lanes' capacities together make
-// enough work for two more launches and the fused form, a block per row, is no better. us, fused ->
-// segments: 31 lanes x 3 rows x 4,000 slots 98 -> 91, ragged 81 -> 70; 31 x 2 x 4,000 99 -> 87; 64 x 2 x
-// 4,000 125 -> 145, 32 x 3 x 3,000 79 -> 87, 31 x 3 x 1,000 42 -> 43. Split path -> segments: 24 x 3 x
-// 8,192 277 -> 127, 16 x 3 x 2,000 65 -> 50, 8 x 3 x 4,000 61 -> 48, 8 x 3 x 2,000 44 -> 45; two rows (the
-// split path reads the K/V only twice then): 24 x 2 x
-// 8,192 186 -> 119, 3 x 2 x 32,768 124 -> 93, 16 x 2 x 2,000 50 -> 56, 8 x 2 x 4,000 49 -> 56.
+// Verify rows by segments where the rows form is not taken and there are slots enough for two more
+// launches; by the lanes' contexts, not their capacity, which may be mostly empty. us, all with another
+// layer's K/V from call to call. Split path -> segments, three rows: 3 lanes x 8,192 slots 62 -> 52, 5 x
+// 4,096 57 -> 48, 8 x 2,000 47 -> 48, 8 x 500 35 -> 43, 3 x 4,096 46 -> 47, 16 x 1,000 48 -> 49, 31 x 500 53 -> 45,
+// 24 x 8,192 297 -> 125. Two rows (the split path reads the K/V only twice then): 16 x 3,000 62 -> 62, 16 x
+// 4,000 74 -> 65, 22 x 4,000 ragged 65 -> 68, 31 x 2,000 78 -> 66, 31 x 1,000 56 -> 59, 48 x 500 51 -> 53, 80 x 500
+// 65 -> 60. One lane's P.V segments are few blocks and its parts' sum is as long as the split path's:
+// 500 slots 33 -> 42, 32,768 84 -> 86, 65,536 154 -> 160. Fused form, a block per row, -> segments: 31 lanes x
+// 3 rows x 1,000 50 -> 55, 1,500 59 -> 61, 2,000 69 -> 64, 4,000 106 -> 91; 32 x 2 x 2,000 70 -> 66, 40 x 2 x 2,000
+// 74 -> 77, 2,500 84 -> 81.
 static bool use_seg(const AttnArgs& a) {
-    if (a.force != kAttnAuto || (a.T != 2 && a.T != 3) || a.R % a.T || use_rows(a)) return false;
-    if (use_fused(a) && (a.R >= 96 || a.cap < 2048)) return false;
-    return (long long)(a.R / a.T) * a.cap >= (a.T == 2 ? 90000 : 30000);
+    if (a.force != kAttnAuto || (a.T != 2 && a.T != 3) || a.R % a.T || a.R == a.T || use_rows(a)) return false;
+    if (a.R >= 192 && uneven(a)) return true;
+    if (use_fused(a)) return a.R < 96 && a.ctx_max >= (a.T == 2 ? 2048 : 1536);
+    return a.T == 2 ? a.ctx_sum + 200ll * a.R >= 54000 : a.ctx_sum + 150ll * a.R >= 18000;
 }
 static bool use_prompt(const AttnArgs& a) {
     const bool shape = a.T >= 64 && a.R == a.T;
@@ -1717,6 +1727,7 @@ hipError_t launch_attn_prep(const AttnArgs& a, hipStream_t st) {
 
 hipError_t launch_attn_core(const AttnArgs& a, hipStream_t st) {
     if (a.R <= 0 || a.max_chunks <= 0) return hipErrorInvalidValue;
+    if (a.T > 1 && (a.ctx_max <= 0 || a.ctx_max > a.cap)) return hipErrorInvalidValue;
     const int lds_slots = (a.cap + 63) / 64 * 64;
     const size_t lds = fused_lds(a);
     if (!attn_form_ok(a)) return hipErrorInvalidValue;
@@ -1735,8 +1746,9 @@ hipError_t launch_attn_core(const AttnArgs& a, hipStream_t st) {
         Q35_ROWS(2, 8) Q35_ROWS(3, 8) Q35_ROWS(2, 4) Q35_ROWS(3, 4)
 #undef Q35_ROWS
     } else if (use_seg(a)) {
-        const int pairs = (a.R / a.T * kNkv + 7) / 8 * 8, ns = a.max_chunks;
-        const int np = ((a.cap + kPart - 1) / kPart + kSegParts - 1) / kSegParts;
+        // blocks up to the longest lane's last slot
+        const int pairs = (a.R / a.T * kNkv + 7) / 8 * 8, ns = (a.ctx_max + kChunk - 1) / kChunk;
+        const int np = (a.ctx_max + kPart * kSegParts - 1) / (kPart * kSegParts);
         const size_t lp = np > 1 ? (size_t)kSegParts * a.T * 4096 : 0;
 #define Q35_SEG(TV)                                                                                              \
     if (a.T == TV) {                                                                                             \
@@ -1764,18 +1776,21 @@ hipError_t launch_attn_core(const AttnArgs& a, hipStream_t st) {
             hipLaunchKernelGGL((attn_fused<false, 1, false>), grid, dim3(256), lds, st, a, lds_slots);
         }
     } else {
+        // chunks that can hold a row's slots (with one row per lane all of the capacity's: a captured step's
+        // positions move on)
+        const int nc = a.T > 1 ? (a.ctx_max + kChunk - 1) / kChunk : a.max_chunks;
         if (a.force == kAttnSplit4 || (a.force != kAttnSplit && a.split4)) {
             if (prep_folded(a))
-                hipLaunchKernelGGL(attn_scores4<true>, dim3(a.R, kNkv, a.max_chunks * 4), dim3(256), 0, st, a);
+                hipLaunchKernelGGL(attn_scores4<true>, dim3(a.R, kNkv, nc * 4), dim3(256), 0, st, a);
             else
-                hipLaunchKernelGGL(attn_scores4<false>, dim3(a.R, kNkv, a.max_chunks * 4), dim3(256), 0, st, a);
-            hipLaunchKernelGGL(attn_pv4, dim3(a.R, kNkv, a.max_chunks * 8), dim3(64), 0, st, a);
+                hipLaunchKernelGGL(attn_scores4<false>, dim3(a.R, kNkv, nc * 4), dim3(256), 0, st, a);
+            hipLaunchKernelGGL(attn_pv4, dim3(a.R, kNkv, nc * 8), dim3(64), 0, st, a);
         } else {
             if (prep_folded(a))
-                hipLaunchKernelGGL(attn_scores_prep, dim3(a.R, kNkv, a.max_chunks * 4), dim3(64), 0, st, a);
+                hipLaunchKernelGGL(attn_scores_prep, dim3(a.R, kNkv, nc * 4), dim3(64), 0, st, a);
             else
-                hipLaunchKernelGGL(attn_scores, dim3(a.R, kNkv, a.max_chunks * 4), dim3(64), 0, st, a);
-            hipLaunchKernelGGL(attn_pv, dim3(a.R, kNkv, a.max_chunks * 2), dim3(256), 0, st, a);
+                hipLaunchKernelGGL(attn_scores, dim3(a.R, kNkv, nc * 4), dim3(64), 0, st, a);
+            hipLaunchKernelGGL(attn_pv, dim3(a.R, kNkv, nc * 2), dim3(256), 0, st, a);
         }
         hipLaunchKernelGGL(attn_combine, dim3(a.R, kNq), dim3(256), 0, st, a, 0);
     }

@@ -611,19 +611,26 @@ void resid_gemm(q35_engine* e, B1Res* rr, const uint16_t* W, int K, int R, const
     }
 }
 
-// Whether no lane occurs twice among the staged rows (T rows per lane): callers of the op and of
-// mtp_draft may name a lane more than once.
-int lanes_distinct(const q35_engine* e, int lanes, int R, int T) {
+// What the attention dispatch knows of the staged rows (T per lane): whether no lane occurs twice
+// (callers of the op and of mtp_draft may name a lane more than once), and the cached slots, the new rows'
+// included, of the longest lane and of all lanes together.
+struct RowSpan { int distinct = 1, ctx_max = 0; long long ctx_sum = 0; };
+RowSpan row_span(const q35_engine* e, int lanes, int R, int T) {
+    RowSpan sp;
     std::vector<char> seen(lanes, 0);
     for (int r = 0; r < R; r += T) {
-        if (seen[e->h_lane[r]]) return 0;
+        if (seen[e->h_lane[r]]) sp.distinct = 0;
         seen[e->h_lane[r]] = 1;
+        const int n = e->h_slot[r + T - 1] + 1;
+        sp.ctx_max = std::max(sp.ctx_max, n);
+        sp.ctx_sum += n;
     }
-    return 1;
+    return sp;
 }
 
 void attention_layer(q35_engine* e, const LayerW& w, int R, uint16_t* kc, uint16_t* vc,
-                     long long kv_lane, long long layer_off, int cap, int distinct, int T = 1, B1Res* rr = nullptr) {
+                     long long kv_lane, long long layer_off, int cap, const RowSpan& span, int T = 1,
+                     B1Res* rr = nullptr) {
     if (small_rows(R))
         norm_gemm(e, rr, w.W_in, kAttnInRows, R, e->proj, kAttnInRows, w.norm_in);
     else
@@ -640,7 +647,7 @@ void attention_layer(q35_engine* e, const LayerW& w, int R, uint16_t* kc, uint16
     a.split4 = e->forms.attn_split4;
     a.fused_pair = e->forms.attn_pair;
     a.rows_form = e->forms.attn_rows;
-    a.distinct = distinct;
+    a.distinct = span.distinct; a.ctx_max = span.ctx_max; a.ctx_sum = span.ctx_sum;
     // a prompt wave's o_proj in the many-row full-K form: attn_prompt writes its output tiled
     const bool tiled = !rr && wide_fullk(e->forms, R) && attn_prompt_form(a);
     a.out_tiled = tiled ? 1 : 0;
@@ -708,7 +715,7 @@ void body_kernels(q35_engine* e, q35_state* s, int R, int T, bool ckpt, int defe
     B1Res res{e->x, e->h};          // one-row bodies: e->h is the second residual buffer
     res.mid = mid_partials(e, R);   // 2 .. 16 rows: e->x folded in place, e->h the normed rows
     B1Res* rr = b1_partials(e, R, T, ckpt) || res.mid ? &res : nullptr;
-    const int distinct = lanes_distinct(e, s->lanes, R, T);
+    const RowSpan span = row_span(e, s->lanes, R, T);
     HCK(launch_addnorm(0, e->tok_dev, e->E, e->x, nullptr, nullptr, 0, e->L[0].norm_in, small ? nullptr : e->h,
                        R, e->st, !small && wide_for(e, R, in_rows(0))));
     for (int l = 0; l < e->n_layers; ++l) {
@@ -756,7 +763,7 @@ void body_kernels(q35_engine* e, q35_state* s, int R, int T, bool ckpt, int defe
                 resid_gemm(e, rr, w.W_out, 2048, R, e->o, 2048, kAGatedNorm, e->proj + kGdnZOff, kGdnInRows, w.gnorm);
         } else {
             attention_layer(e, w, R, s->kc, s->vc, s->kv_lane(),
-                            (long long)attn_slot(l) * 2 * s->capT * 256, s->capT, distinct, T, rr);
+                            (long long)attn_slot(l) * 2 * s->capT * 256, s->capT, span, T, rr);
         }
         mlp_layer(e, w, R, rr);
         const bool lastl = l + 1 == e->n_layers;
@@ -815,7 +822,7 @@ void mtp_draft_pass(q35_engine* e, q35_state* s, int n, const uint16_t* hsrc) {
         HCK(launch_addnorm(4, nullptr, nullptr, e->x, nullptr, e->kpart, gemm_partial_chains(n, 2048, e->forms), e->M.norm_in, e->h, n, e->st,
                            wide_for(e, n, kAttnInRows)));
     }
-    attention_layer(e, e->M, n, s->mkc, s->mvc, s->mkv_lane(), 0, s->mtp_capT, lanes_distinct(e, s->lanes, n, 1));
+    attention_layer(e, e->M, n, s->mkc, s->mvc, s->mkv_lane(), 0, s->mtp_capT, row_span(e, s->lanes, n, 1));
     mlp_layer(e, e->M, n);
     finish_norm(e, n, e->mtp_norm, e->nrm);
 }
@@ -1903,7 +1910,8 @@ int q35_op_attn_decode(q35_engine* e, q35_state* s, int layer, const int32_t* la
         a.out = out; a.R = R; a.T = T; a.inv_freq = e->inv_freq; a.prompt_flash = e->forms.attn_prompt;
         a.split4 = e->forms.attn_split4; a.fused_pair = e->forms.attn_pair; a.rows_form = e->forms.attn_rows;
         a.force = form;
-        a.distinct = lanes_distinct(e, s->lanes, R, T);
+        const RowSpan span = row_span(e, s->lanes, R, T);
+        a.distinct = span.distinct; a.ctx_max = span.ctx_max; a.ctx_sum = span.ctx_sum;
         REQ(attn_form_ok(a), Q35_ERR_ARG, "this attention form cannot run this shape (rows, rows per lane, capacity)");
         HCK(launch_attn_prep(a, e->st));
         HCK(launch_attn_core(a, e->st));

@@ -23,7 +23,7 @@ struct KernelForms {
     int partial_rows = 1024;   // batched kEPartial GEMMs with M >= this leave one (summed) chain
     int attn_split4 = 1;       // split attention path: 4-wave score blocks, P.V split over dim quarters
     int attn_pair = 1;         // fused attention, one row per lane: two (row, kv head) items per block
-    int attn_rows = 2;         // MTP verify (2-3 rows per lane) from 192 rows on: one block per (lane, kv head)
+    int attn_rows = 2;         // MTP verify (2-3 rows per lane) from 192 rows on, the lanes not too uneven: one block per (lane, kv head)
                                // (1: 4 waves, two blocks per CU; 2: 8 waves, one per CU, a larger LDS tail)
     int attn_prompt = 1;       // prompt waves of >= 64 rows: flash-form MFMA kernel (1) or one-row kernels (0)
     int mid_partials = 1;      // bodies of 2 .. 16 rows: k-block chains + add+norm (0: residual-epilogue GEMMs)
@@ -189,6 +189,10 @@ struct AttnArgs {
     int rows_form;         // KernelForms::attn_rows
     int force;             // 0: the form chosen from the shape; else one form (AttnForce), for
                            // the op-level parity harness; a form the shape cannot take is an error
+    // Cached slots, the new rows' included, of the longest lane and of all lanes together. For T > 1
+    // only: a captured step (always T = 1) is replayed at later positions than these.
+    int ctx_max;
+    long long ctx_sum;
 };
 enum AttnForce { kAttnAuto = 0, kAttnSplit = 1, kAttnSplit4 = 2, kAttnFused = 3, kAttnFusedPair = 4,
                  kAttnRows = 5, kAttnPrompt = 6 };

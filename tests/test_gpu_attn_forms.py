@@ -71,27 +71,71 @@ def test_folded_prep_equals_split(harness, B, T):
 
 @pytest.mark.parametrize("T", [2, 3])
 def test_segments_equal_split(T):
-    """Verify rows of 31 lanes x 3,000 slots (the segment form) at the borders of its chunks (256
-    slots) and P.V segments (512), rows that straddle them, a lane of one segment and an empty one,
-    and with a lane named twice (q and K / V rows from the prep launch)."""
-    h = Harness(3000, 128)
+    """Verify rows of 31 lanes (the segment form) at the borders of its chunks (256 slots) and P.V
+    segments (512), rows that straddle them, a lane of one segment and an empty one, some of 7,000
+    slots and more, and with a lane named twice (q and K / V rows from the prep launch)."""
+    h = Harness(8192, 128)
     try:
         pos = [0, 1, 62, 126, 253, 254, 255, 256, 509, 510, 511, 512, 513, 1022, 1023, 1024, 1535, 2047, 2048, 2303,
-               2558, 2815, 2990, 3000 - T]
-        pos += [int(p) for p in np.random.default_rng(T).integers(0, 2990, 7)]
+               2558, 2815, 4095, 8192 - T]
+        pos += [int(p) for p in np.random.default_rng(T).integers(7000, 8190, 7)]
         lanes = np.random.default_rng(T).permutation(256)[:31].tolist()
         want = h.run(lanes, pos, T, 1)
         for i in range(31):
-            for n in "kv":
-                full = np.asarray(h.s.read(lanes[i], n, pos[i] + T))
-                full[LAYER][:, pos[i]:pos[i] + T] = 0
-                h.s.write(lanes[i], n, full, pos[i] + T)
+            clear_slots(h, lanes[i], pos[i], T)
+        before = prepared_q(h)
         assert np.array_equal(h.run(lanes, pos, T, 0), want)
+        assert np.array_equal(h.e.read_scratch("q", (2048,), np.float32), before)
         for i in (0, 6, 11, 23):
             h.check_lane(i, lanes[i], pos[i], T, want)
         lanes[5] = lanes[6]                 # a second group of the lane, right after the first
         pos[5] = pos[6] + T
-        assert np.array_equal(h.run(lanes, pos, T, 0), h.run(lanes, pos, T, 1))
+        rest = [i for i in range(31) if i != 5]
+        clear_slots(h, lanes[6], pos[6], 2 * T)
+        first = h.run(lanes, [p if i != 5 else 8000 for i, p in enumerate(pos)], T, 1)   # group 5 elsewhere for now
+        last = run_from(h, 5 * T, [lanes[5]], [pos[5]], T, 1)
+        clear_slots(h, lanes[6], pos[6], 2 * T)
+        before = prepared_q(h)
+        got = h.run(lanes, pos, T, 0).reshape(31, T, 2048)
+        assert not np.array_equal(h.e.read_scratch("q", (2048,), np.float32), before)
+        assert np.array_equal(got[rest], first.reshape(31, T, 2048)[rest])
+        assert np.array_equal(got[5], last)
+    finally:
+        h.s.close()
+        h.e.close()
+
+
+@pytest.mark.parametrize("T", [2, 3])
+def test_few_long_lanes_equal_split(T):
+    """100 lanes of which one has 8,000 slots and the others at most 1,000: by segments (in the rows
+    form the long lane's block would run alone), the same bits as the split form and the rows form."""
+    h = Harness(8192, 300)
+    try:
+        pos = [8000] + [int(p) for p in np.random.default_rng(T).integers(0, 1000, 99)]
+        lanes = np.random.default_rng(T).permutation(256)[:100].tolist()
+        want = h.run(lanes, pos, T, 1)
+        for form in (0, 5):
+            for i in range(0, 100, 9):
+                clear_slots(h, lanes[i], pos[i], T)
+            assert np.array_equal(h.run(lanes, pos, T, form), want), form
+    finally:
+        h.s.close()
+        h.e.close()
+
+
+@pytest.mark.parametrize("lanes, ctx, T, segments", [
+    (1, 500, 3, False), (1, 4096, 3, False), (3, 500, 3, False), (3, 4096, 2, False), (8, 500, 3, False), (8, 4096, 3, True),
+    (4, 16000, 2, True), (24, 500, 2, False)])
+def test_form_by_context_not_capacity(lanes, ctx, T, segments):
+    """A state of 16,384 slots per lane: verify rows go by the slots in use (segments make q in their
+    blocks; the split path's comes from the prep launch), and the bits are the split path's."""
+    h = Harness(16384, 128)
+    try:
+        pos = [ctx - T - 7 * i for i in range(lanes)]
+        before = prepared_q(h)
+        got = h.run(list(range(lanes)), pos, T, 0)
+        assert np.array_equal(h.e.read_scratch("q", (2048,), np.float32), before) == segments
+        assert np.array_equal(got, h.run(list(range(lanes)), pos, T, 1))
     finally:
         h.s.close()
         h.e.close()
