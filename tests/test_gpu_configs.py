@@ -230,22 +230,24 @@ def test_config3_attention_batched(oracle_weights, B, L):
     e.close()
 
 
-def test_attention_two_items_per_block_bit_identical():
-    """One row per lane at batched lanes runs two (row, kv head) items per attention block
+@pytest.mark.parametrize("cap", [1000, 4096])
+def test_attention_two_items_per_block_bit_identical(cap):
+    """One row per lane above 128 lanes runs two (row, kv head) items per attention block
     (engine option attn_pair). With ragged contexts (lanes l and l + 4, which share a block,
     alternate between 300 and 900 cached slots, so the halves run different part counts) and
-    100 lanes (the last block has idle halves), logits and tokens equal the one-item blocks'
-    bit for bit."""
+    150 lanes (the last blocks have idle halves), logits and tokens equal the one-item blocks'
+    bit for bit, with q and the K / V rows made in the blocks (150 x 1,000 slots) and by the prep
+    launch (150 x 4,096)."""
     from qwen35 import Engine, State
-    print("attention two items per block", flush=True)
-    B = 100
-    e = Engine(max_rows=128, max_ctx=1024, seed=0, use_graph=False)
+    print(f"attention two items per block, capacity {cap}", flush=True)
+    B = 150
+    e = Engine(max_rows=160, max_ctx=cap + 24, seed=0, use_graph=False)
     try:
         toks = [int(t) for t in np.random.default_rng(5).integers(0, 248320, B)]
         outs = []
         for pair in (1, 0):
             e.set_option("attn_pair", pair)
-            short, long_ = State(e, B, 1000), State(e, B, 1000)
+            short, long_ = State(e, B, cap), State(e, B, cap)
             short.seed(3, 300)
             long_.seed(4, 900)
             for ln in range(B):
