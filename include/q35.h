@@ -246,9 +246,9 @@ int q35_kprof_read(q35_engine* e, float* total_ms, int* launches);
  * switches of this engine only (each engine holds its own; setting one drops the engine's
  * captured steps), each bit-identical to its alternative and kept for A/B measurement:
  * "b1_partials" (one-row bodies leave k-block chains for the next norm GEMV), "gemv_tpb" (1/2
- * column tiles per block of the one-row norm GEMVs), "gemm_pre" (batched K = 1024 GEMMs; 0: k-block
- * pipelined, 1: all loads issued up front, in 64 x 128 blocks when those fit the CUs in one
- * round, else 32 x 64; 2: always 64 x 128), "lmhead_persist" (lm_head at batched lanes: 0 tiled, 1 persistent with A in LDS, 3 -- the
+ * column tiles per block of the one-row norm GEMVs), "gemm_pre" (batched K = 1024 GEMMs of
+ * row-major A; 0: k-block pipelined, 1: an LDS ring in 64 x 128 blocks where their rounds are well
+ * filled, else all loads issued up front in 32 x 64 blocks; 2: all up front in 64 x 128), "lmhead_persist" (lm_head at batched lanes: 0 tiled, 1 persistent with A in LDS, 3 -- the
  * default -- persistent with A in registers and a running argmax per column stream), "partial_rows"
  * (>= 17: batched out/o/down GEMMs with at least this many rows sum their k-block chains in
  * the block, one chain for the add+norm; default 1,024), "attn_split4" (split attention path

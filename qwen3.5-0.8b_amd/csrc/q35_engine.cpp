@@ -539,7 +539,8 @@ inline bool small_rows(int R) { return R <= 16; }
 // fragment layout (the producing add+norm writes e->h so) and runs gemm_wide: bodies of >= 512
 // rows (prompt waves, MTP verify at many lanes, 256-row tiles) and batched lanes of 17 .. 511
 // rows (64-row tiles) except the GDN in_proj, whose 65 column blocks x 4 row blocks at 256 rows
-// would not fit the 256 CUs in one round (gemm_pre instead: 13.9 against 13.7 us in two rounds).
+// would not fit the 256 CUs in one round (row-major A instead: gemm_pre there, 13.9 against 13.7 us in
+// two rounds; gemm_rows64 at lane counts that fill its rounds).
 inline bool wide_for(const q35_engine* e, int R, int N) {
     return e->forms.gemm_wide && R > 16 && (R >= 512 || N != kGdnInRows);
 }

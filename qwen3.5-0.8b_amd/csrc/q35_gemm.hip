@@ -1726,6 +1726,8 @@ static void launch_large(const GemmArgs& a, hipStream_t st) {
         hipLaunchKernelGGL((gemm_large_m<EM, 4, 16>), dim3((nb16 + 7) / 8 * 8 * mb, 1, gz), dim3(1024), 0, st, a);
         return;
     }
+    const int nb8 = EM == kESiluMul ? (a.N / 32 + 3) / 4 : (a.N / 16 + 7) / 8;   // 64 x 128 blocks
+    const long long b = (long long)nb8 * mb;
     if ((EM == kEStore || EM == kESiluMul) && a.K == kHidden && a.forms.gemm_pre == 1 && rows_ok(a)) {
         // 64 x 128 blocks of gemm_rows64 (8.9 us the first round of 256, 7.8 each further one)
         // unless gemm_pre's smaller blocks, which cost 3.3 us and 8.9 per 256 of those blocks, lose
@@ -1734,7 +1736,6 @@ static void launch_large(const GemmArgs& a, hipStream_t st) {
         // 17.9 / 62.0 (112, 224, 448, 1,792 blocks); qkv (N = 5120) at 256 / 512 / 768 rows 9.6 /
         // 14.5 / 20.6 -> 8.9 / 16.5 / 17.4 (160, 320, 480); in_proj (8224) at 256 / 384 13.4 / 17.5
         // -> 15.9 / 16.7 (260, 390)
-        const long long b = (long long)(EM == kESiluMul ? (a.N / 32 + 3) / 4 : (a.N / 16 + 7) / 8) * mb;
         if (10 * b > 256 * (9 * ((b + 255) / 256) - 3)) {
             launch_rows64<EM == kESiluMul ? kESiluMul : kEStore>(a, st);
             return;
@@ -1744,14 +1745,13 @@ static void launch_large(const GemmArgs& a, hipStream_t st) {
         // 32-row blocks (64 KiB of A fragments: two blocks per CU); 64-row blocks (128 KiB,
         // one per CU) measured 10-35 % slower
         // 64 x 128 blocks of 8 waves (one per CU, half the L2 -> CU bytes per output of the
-        // 32 x 64 tiles) when they fill the CUs in one round: gate|up at 256 lanes, 224 blocks,
-        // 16.8 -> 14.8 us in the model (in_proj's 288 blocks take two rounds: 21.7 us against
-        // 17.0; the attention qkv's 160 blocks leave CUs idle: 12.8 against 12.0); form 2 forces
-        // them (tests)
-        const int nb8 = EM == kESiluMul ? (a.N / 32 + 3) / 4 : (a.N / 16 + 7) / 8, mb4 = (a.M + 63) / 64;
-        const int grid8 = (nb8 + 7) / 8 * 8 * mb4;
-        if (a.forms.gemm_pre == 2 || (grid8 <= 256 && 4 * grid8 > 3 * 256)) {
-            hipLaunchKernelGGL((gemm_pre<EM, 4, 8>), dim3(grid8), dim3(512), pre_lds_bytes<4>(), st, a);
+        // 32 x 64 tiles) when they fill the CUs in one round (gate|up at 256 rows, 224 blocks, cold
+        // weights: 16.8 -> 14.8 us; 288 blocks take two rounds, 17.0 -> 21.7, 160 leave CUs idle,
+        // 12.0 -> 12.8): operands that rows_ok excludes, gemm_rows64 has the others. Blocks with columns
+        // are counted, not the launched multiple of 8 columns of blocks (N = 128 at 2,048 rows, 32
+        // of 256: 10.4 us, 7.4 in 32-row blocks). Form 2 forces them (tests).
+        if (a.forms.gemm_pre == 2 || (b <= 256 && 4 * b > 3 * 256)) {
+            hipLaunchKernelGGL((gemm_pre<EM, 4, 8>), dim3((nb8 + 7) / 8 * 8 * mb), dim3(512), pre_lds_bytes<4>(), st, a);
             return;
         }
         const int mb2 = (a.M + 31) / 32;

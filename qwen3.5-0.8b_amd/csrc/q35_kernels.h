@@ -16,7 +16,8 @@ enum { kEStore = 0, kEArgmax = 1, kEPartial = 2, kEResidual = 3, kESiluMul = 4 }
 // with the launch arguments, so engines of one process never see each other's settings.
 struct KernelForms {
     int gemv_tpb = 2;          // one-row norm GEMVs (N >= 4096): column tiles per block, 1 or 2
-    int gemm_pre = 1;          // batched K = 1024 GEMMs: all loads up front (1) or k-block pipelined (0)
+    int gemm_pre = 1;          // batched K = 1024 GEMMs of row-major A: an LDS ring where its blocks fill the
+                               // CUs, else all loads up front (1; 2: always these, 64 x 128), or k-block pipelined (0)
     int lmhead_persist = 3;    // tied lm_head at batched lanes: 64 x 256 tiles (0), persistent with A in LDS
                                // (1), persistent with A in registers, the weights through an LDS ring
                                // and one argmax partial per (row, column stream) (3)

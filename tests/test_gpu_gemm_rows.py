@@ -23,7 +23,7 @@ def eng():
     (16, 4096, 40, 0), (48, 4096, 31, 0), (272, 1280, 65, 0), (1024, 256, 100, 0), (1024, 256, 900, 0),
     (1008, 512, 1100, 8), (4112, 768, 300, 0), (2048, 2304, 1000, 0),
     # K = 1024: either side of the line between the 32 x 64 and the 64 x 128 blocks (153 of 256)
-    (5120, 1024, 192, 0), (5120, 1024, 256, 8), (7168, 1024, 449, 0), (8224, 1024, 384, 0), (2064, 1024, 600, 0)])
+    (5120, 1024, 192, 0), (5120, 1024, 256, 8), (7168, 1024, 449, 0), (8224, 1024, 384, 0), (2064, 1024, 600, 0), (128, 1024, 2048, 0)])
 def test_row_major_gemm_equals_one_tile_kernel(eng, N, K, M, pad):
     import torch
     print(f"rows gemm N={N} K={K} M={M} ldx={K + pad}", flush=True)
